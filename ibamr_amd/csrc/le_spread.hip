@@ -132,7 +132,10 @@ struct SpreadArgs
     int dom_lo[3], dom_hi[3];
     int pshift[3];
     double dx[3];
-    double vol;
+    double rdx[3];  // FP64: 1 / dx
+    int dx_ok;      //       dx in div_by's range
+    double vol, rvol;
+    int vol_div;   // FP64: 1: vol is a power of two, 2: quotients by vol from its reciprocal (div_by), 0: divisions
     int fdepth;
     int narr;
     int gcw[3];
@@ -434,6 +437,7 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
     a.F = static_cast<const T*>(F);
     a.cells = P->cell_sorted_d;
     a.bin_start = P->bin_start_d;
+    a.dx_ok = 1;
     for (int d = 0; d < 3; ++d)
     {
         a.nb[d] = P->nb[d];
@@ -442,10 +446,17 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
         a.dom_hi[d] = P->dom_hi[d];
         a.pshift[d] = P->pshift[d];
         a.dx[d] = P->dx[d];
+        a.rdx[d] = 1.0 / P->dx[d];
+        if (P->dx[d] < 1e-60 || P->dx[d] > 1e60) a.dx_ok = 0;
         a.gcw[d] = P->data_gcw[d];
     }
     a.bin = P->bin;
     a.vol = P->ndim == 3 ? (P->dx[0] * P->dx[1]) * P->dx[2] : P->dx[0] * P->dx[1];
+    {
+        int e;
+        a.rvol = 1.0 / a.vol;
+        a.vol_div = a.vol < 1e-60 || a.vol > 1e60 ? 0 : (std::frexp(a.vol, &e) == 0.5 ? 1 : 2);
+    }
     a.fdepth = P->fdepth;
     a.narr = P->narr;
     a.idx_gcw = P->idx_gcw;
@@ -461,7 +472,8 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
 // Spread tile shapes built for each form; the first is the default.
 //   2-D: a 16 x 16 tile in LDS (k_spread_tiles).
 //   3-D: 8 x 8 or 16 x 4 grid lines (one per lane) times a column of z values
-//     in registers (k_spread3); FP32C keeps two register sets per z value (the
+//     in registers (k_spread3b FP64, k_spread3 FP32C); an FP64 tile is cut along z
+//     into work items (spread_cut).  FP32C keeps two register sets per z value (the
 //     FP64 total and the chunk's FP32 partial), so its columns are shorter.
 //     FP32C z extents of SWEEP_MIN_Z or more are z segments swept through a
 //     register window (k_spread3s).
@@ -499,6 +511,42 @@ bool shape_admissible(const ibamr_plan* P, const Shape& sh)
     return !sweep || n[0] * n[1] <= 64;
 }
 
+// Tiles of the given extents over every array of every patch (one depth component).
+long count_tiles(const ibamr_plan* P, const Shape& ext)
+{
+    long total = 0;
+    for (const PatchDev& pd : P->patches_h)
+        for (int a = 0; a < P->narr; ++a)
+        {
+            long t = 1;
+            for (int d = 0; d < P->ndim; ++d)
+            {
+                const int n = pd.ihi[d] - pd.ilo[d] + 1 + 2 * P->data_gcw[d] +
+                              (P->centering == IBAMR_SIDE && d == a ? 1 : 0);
+                t *= (n + ext[d] - 1) / ext[d];
+            }
+            total += t;
+        }
+    return total;
+}
+
+// z extent of a shape's work items (k_spread3b; the results do not depend on it).
+// A wavefront takes its tile's points one after another, so the tiles along a
+// dense surface are the critical path: 16 values each beat 32 everywhere (256^3
+// IB_4, 10^6 points on a shell: 1.18 against 1.79 ms; AMR level of 384^3 0.79
+// against 1.08 ms).  Fewer tiles than the GPU holds wavefronts (256 CUs x 16):
+// 8 values (40^3, 432 tiles: 29 against 40 us; 64^3 IB_6, 1568 tiles: 259 against
+// 357 us; at 8736 tiles 207 against 185 us).  More than 128 per SIMD: 24, which
+// visit a point in fewer tiles (512^3 IB_6: 9.4 against 10.5 ms; at 86 k tiles
+// 1.35 against 1.11 ms).
+int spread_cut(const ibamr_plan* P, const Shape& sh)
+{
+    if (P->ndim != 3 || P->precision != IBAMR_FP64) return sh[2];
+    if (sh[0] != 8 || sh[2] != 32) return 16;
+    if (count_tiles(P, {8, 8, 16}) < 4096) return 8;
+    return count_tiles(P, {8, 8, 24}) >= (1L << 17) ? 24 : 16;
+}
+
 // Work list of one tile shape: every tile of every array of every patch.
 // XCD-aware launch order: workgroup i runs on XCD i % 8.  Tiles are grouped by
 // (patch, z row, y row), each group holding that row of every array, and the
@@ -511,6 +559,8 @@ bool shape_admissible(const ibamr_plan* P, const Shape& sh)
 int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
 {
     std::vector<TileDesc> tiles;
+    const Shape ext = {sh[0], sh[1], spread_cut(P, sh)};
+    out.cut = ext[2];
     const int ncomp_tiles = P->centering == IBAMR_SIDE ? P->ndim : P->depth;
     std::vector<std::vector<TileDesc>> q(8);
     size_t g = 0;
@@ -525,7 +575,7 @@ int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
             for (int d = 0; d < P->ndim; ++d)
             {
                 const int n = pd.ihi[d] - pd.ilo[d] + 1 + 2 * P->data_gcw[d] + (d == axis ? 1 : 0);
-                nt[c][d] = (n + sh[d] - 1) / sh[d];
+                nt[c][d] = (n + ext[d] - 1) / ext[d];
                 mt[d] = std::max(mt[d], nt[c][d]);
             }
         }
@@ -655,9 +705,19 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
     }
             if constexpr (sizeof(T) == 8)
             {
-                IBAMR_S3(8, 32)
-                IBAMR_S3(8, 16)
-                IBAMR_S3(16, 32)
+#define IBAMR_S3B(TX, ZC)                                                      \
+    if (tl.shape[0] == TX && tl.cut == ZC)                                     \
+    {                                                                          \
+        hipLaunchKernelGGL((k_spread3b<KER, ZC, TX>), G, B, 0, s, a);          \
+        HIP_OK(hipGetLastError());                                             \
+        if (t_end) HIP_OK(hipEventRecord(t_end, s));                           \
+        return IBAMR_OK;                                                       \
+    }
+                IBAMR_S3B(8, 24)
+                IBAMR_S3B(8, 16)
+                IBAMR_S3B(8, 8)
+                IBAMR_S3B(16, 16)
+#undef IBAMR_S3B
             }
             else
             {

@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace ibamr
 {
 enum KernelId : int
@@ -89,6 +91,36 @@ struct KernelTraits<K_PWL>
 // Fortran NINT: round half away from zero.
 __device__ __forceinline__ int nint_d(double x) { return (int)round(x); }
 
+// a / b rounded once, b > 0 with y = 1 / b rounded once: two Newton corrections of
+// a y with exact remainders (Markstein: correcting a quotient within one unit of
+// the last place once more rounds it correctly).  For operands whose remainders
+// neither overflow nor underflow; a zero keeps its sign.  6 operations instead of
+// the 11 (one of quarter rate) of a division.
+__device__ __forceinline__ double div_by(double a, double b, double y)
+{
+    double q = a * y;
+    q = fma(fma(-b, q, a), y, q);
+    q = fma(fma(-b, q, a), y, q);
+    return copysign(q, a);
+}
+
+// How the FP64 weights form their quotients by dx: a division, or div_by with
+// the reciprocal y of dx (operands out of div_by's range divide; y = 0: all do).
+struct Divide
+{
+    __device__ double operator()(double a, double b) const { return a / b; }
+};
+struct DivideBy
+{
+    double y;
+    __device__ double operator()(double a, double b) const
+    {
+        const double m = fabs(a);
+        if (y != 0.0 && ((m >= 1e-200 && m <= 1e200) || a == 0.0)) return div_by(a, b, y);
+        return a / b;
+    }
+};
+
 // lagrangian_delta.f.m4:243-260, FP64
 __device__ __forceinline__ double bspline3_delta_d(double x)
 {
@@ -157,11 +189,12 @@ __device__ __forceinline__ double bspline6_delta_d(double x)
 // Shared stencil of BSPLINE_4/5/6: centre cell of X+Xshift, then the odd order
 // takes centre -2..+2 and the even orders one side chosen by comparing the
 // unshifted X with that cell's centre (Xu; Xu = Xs without a shift).
-template <int K>
-__device__ __forceinline__ int bspline_hi_weights(double Xs, double Xu, double x_lower, double dx, double* w)
+template <int K, typename Q = Divide>
+__device__ __forceinline__ int bspline_hi_weights(double Xs, double Xu, double x_lower, double dx, double* w,
+                                                  Q quot = Q{})
 {
     constexpr int W = KernelTraits<K>::W;
-    const int c = (int)floor((Xs - x_lower) / dx);
+    const int c = (int)floor(quot(Xs - x_lower, dx));
     int lo;
     if (K == K_BS5)
         lo = c - 2;
@@ -174,10 +207,28 @@ __device__ __forceinline__ int bspline_hi_weights(double Xs, double Xu, double x
     for (int k = 0; k < W; ++k)
     {
         const double X_cell = x_lower + ((double)(lo + k) + 0.5) * dx;
-        const double t = (Xs - X_cell) / dx;
+        const double t = quot(Xs - X_cell, dx);
         w[k] = K == K_BS4 ? bspline4_delta_d(t) : (K == K_BS5 ? bspline5_delta_d(t) : bspline6_delta_d(t));
     }
     return lo;
+}
+
+// A stencil of W values starting at lo (relative to ilower) reaches an index i of
+// [f, l] when t = (Xs - x_lower) / dx lies in [f + reach_lo, l + reach_hi] (closed
+// and a little wide: for tests before the weights are evaluated).
+// IB_4/IB_6: lo = nint(t) - W/2; BSPLINE_3/5: floor(t) - (W-1)/2; PIECEWISE_LINEAR:
+// floor(t - 1/2); BSPLINE_4/6: floor(t) - W/2 or one more.
+template <int K>
+constexpr double reach_lo()
+{
+    constexpr int W = KernelTraits<K>::W;
+    return (KernelTraits<K>::IB ? -W / 2 + 0.5 : K == K_PWL ? -0.5 : W % 2 ? -(W - 1) / 2 : -W / 2) - 1e-6;
+}
+template <int K>
+constexpr double reach_hi()
+{
+    constexpr int W = KernelTraits<K>::W;
+    return (KernelTraits<K>::IB ? W / 2 + 0.5 : K == K_PWL ? 1.5 : W % 2 ? (W + 1) / 2 : W / 2 + 1) + 1e-6;
 }
 
 // K of the 6-point kernel (f.m4:2227) and the constant sub-expressions of
@@ -198,7 +249,8 @@ __device__ __forceinline__ IB6Const ib6_const()
     return c;
 }
 
-__device__ __forceinline__ void ib6_weights_d(double r, double* w)
+template <typename Q>
+__device__ __forceinline__ void ib6_weights_d(double r, double* w, Q)
 {
     const IB6Const c = ib6_const();
     const double K = c.K;
@@ -210,7 +262,12 @@ __device__ __forceinline__ void ib6_weights_d(double r, double* w)
     const double beta = (((9.0 / 4.0) - (3.0 / 2.0) * (K + r2)) + c.c_b1 * r) - (7.0 / 3.0) * r3;
     const double gamma = (1.0 / 4.0) * ((c.c_g1 * r2 + c.c_g2 * r4) + (5.0 / 18.0) * r6);
     const double discr = beta * beta - (4.0 * alpha) * gamma;
-    const double pm3 = (-beta + 1.0 * sqrt(discr)) / (2.0 * alpha); // sign(1, 3/2-K) = +1
+    const double num = -beta + 1.0 * sqrt(discr);  // sign(1, 3/2-K) = +1
+    double pm3;
+    if constexpr (std::is_same<Q, Divide>::value)
+        pm3 = num / (2.0 * alpha);
+    else
+        pm3 = DivideBy{1.0 / 56.0}(num, 56.0);
     w[0] = pm3;
     w[1] = ((((-(3.0 * pm3)) - (1.0 / 16.0)) + (1.0 / 8.0) * (K + r2)) + c.c_m2 * r) + (1.0 / 12.0) * r3;
     w[2] = (((2.0 * pm3) + (1.0 / 4.0)) + c.c_m1 * r) - (1.0 / 6.0) * r3;
@@ -250,82 +307,69 @@ __device__ __forceinline__ void ib6_weights_f(float r, float* w)
     (void)K;
 }
 
-// FP64 1-D weights.  Xs = X + Xshift (already added, as the Fortran does);
-// returns the first stencil index relative to ilower.
-template <int K>
-__device__ __forceinline__ int weights_1d(double Xs, double x_lower, double dx, double* w);
-
-template <>
-__device__ __forceinline__ int weights_1d<K_IB4>(double Xs, double x_lower, double dx, double* w)
+// FP64 1-D weights.  Xs = X + Xshift (already added, as the Fortran does); Xu = X
+// (BSPLINE_4/6 choose their side with it); quot forms the quotients by dx.
+// Returns the first stencil index relative to ilower.
+template <int K, typename Q>
+__device__ __forceinline__ int weights_1d_q(double Xs, double Xu, double x_lower, double dx, double* w, Q quot)
 {
-    const double X_o_dx = (Xs - x_lower) / dx;
-    const int lo = nint_d(X_o_dx) - 2;
-    const double r = X_o_dx - ((double)(lo + 1) + 0.5);
-    const double q = sqrt(1.0 + (4.0 * r) * (1.0 - r));
-    w[0] = 0.125 * ((3.0 - 2.0 * r) - q);
-    w[1] = 0.125 * ((3.0 - 2.0 * r) + q);
-    w[2] = 0.125 * ((1.0 + 2.0 * r) + q);
-    w[3] = 0.125 * ((1.0 + 2.0 * r) - q);
-    return lo;
-}
-
-template <>
-__device__ __forceinline__ int weights_1d<K_IB6>(double Xs, double x_lower, double dx, double* w)
-{
-    const double X_o_dx = (Xs - x_lower) / dx;
-    const int lo = nint_d(X_o_dx) - 3;
-    const double r = (1.0 - X_o_dx) + ((double)(lo + 2) + 0.5);
-    ib6_weights_d(r, w);
-    return lo;
-}
-
-template <>
-__device__ __forceinline__ int weights_1d<K_BS3>(double Xs, double x_lower, double dx, double* w)
-{
-    const int c = (int)floor((Xs - x_lower) / dx);
-    const int lo = c - 1;
+    if constexpr (K == K_IB4)
+    {
+        const double X_o_dx = quot(Xs - x_lower, dx);
+        const int lo = nint_d(X_o_dx) - 2;
+        const double r = X_o_dx - ((double)(lo + 1) + 0.5);
+        const double q = sqrt(1.0 + (4.0 * r) * (1.0 - r));
+        w[0] = 0.125 * ((3.0 - 2.0 * r) - q);
+        w[1] = 0.125 * ((3.0 - 2.0 * r) + q);
+        w[2] = 0.125 * ((1.0 + 2.0 * r) + q);
+        w[3] = 0.125 * ((1.0 + 2.0 * r) - q);
+        return lo;
+    }
+    else if constexpr (K == K_IB6)
+    {
+        const double X_o_dx = quot(Xs - x_lower, dx);
+        const int lo = nint_d(X_o_dx) - 3;
+        const double r = (1.0 - X_o_dx) + ((double)(lo + 2) + 0.5);
+        ib6_weights_d(r, w, quot);
+        return lo;
+    }
+    else if constexpr (K == K_BS3)
+    {
+        const int c = (int)floor(quot(Xs - x_lower, dx));
+        const int lo = c - 1;
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-    {
-        const double X_cell = x_lower + ((double)(lo + k) + 0.5) * dx;
-        w[k] = bspline3_delta_d((Xs - X_cell) / dx);
+        for (int k = 0; k < 3; ++k)
+        {
+            const double X_cell = x_lower + ((double)(lo + k) + 0.5) * dx;
+            w[k] = bspline3_delta_d(quot(Xs - X_cell, dx));
+        }
+        return lo;
     }
-    return lo;
-}
-
-template <>
-__device__ __forceinline__ int weights_1d<K_BS4>(double Xs, double x_lower, double dx, double* w)
-{
-    return bspline_hi_weights<K_BS4>(Xs, Xs, x_lower, dx, w);
-}
-template <>
-__device__ __forceinline__ int weights_1d<K_BS5>(double Xs, double x_lower, double dx, double* w)
-{
-    return bspline_hi_weights<K_BS5>(Xs, Xs, x_lower, dx, w);
-}
-template <>
-__device__ __forceinline__ int weights_1d<K_BS6>(double Xs, double x_lower, double dx, double* w)
-{
-    return bspline_hi_weights<K_BS6>(Xs, Xs, x_lower, dx, w);
-}
-
-// PIECEWISE_LINEAR, lagrangian_interaction3d.f.m4:680-699 (spread) / 556-575
-// (interp): the cell whose centre is nearest, then the linear hat on the two
-// cells straddling X.
-template <>
-__device__ __forceinline__ int weights_1d<K_PWL>(double Xs, double x_lower, double dx, double* w)
-{
-    const int c = nint_d((Xs - x_lower) / dx - 0.5);
-    const double X_cell = x_lower + ((double)c + 0.5) * dx;
-    if (Xs < X_cell)
+    else if constexpr (K == K_PWL)
     {
-        w[0] = (X_cell - Xs) / dx;
+        // PIECEWISE_LINEAR, lagrangian_interaction3d.f.m4:680-699 (spread) / 556-575
+        // (interp): the cell whose centre is nearest, then the linear hat on the two
+        // cells straddling X.
+        const int c = nint_d(quot(Xs - x_lower, dx) - 0.5);
+        const double X_cell = x_lower + ((double)c + 0.5) * dx;
+        if (Xs < X_cell)
+        {
+            w[0] = quot(X_cell - Xs, dx);
+            w[1] = 1.0 - w[0];
+            return c - 1;
+        }
+        w[0] = 1.0 + quot(X_cell - Xs, dx);
         w[1] = 1.0 - w[0];
-        return c - 1;
+        return c;
     }
-    w[0] = 1.0 + (X_cell - Xs) / dx;
-    w[1] = 1.0 - w[0];
-    return c;
+    else
+        return bspline_hi_weights<K>(Xs, Xu, x_lower, dx, w, quot);
+}
+
+template <int K>
+__device__ __forceinline__ int weights_1d(double Xs, double x_lower, double dx, double* w)
+{
+    return weights_1d_q<K>(Xs, Xs, x_lower, dx, w, Divide{});
 }
 
 // FP32 1-D weights: index selection and the offset r in FP64, weights in FP32.
