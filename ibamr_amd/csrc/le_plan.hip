@@ -353,20 +353,7 @@ static int plan_create_impl(ibamr_plan** out, const ibamr_level_geom* L, const i
     if (bpl.empty()) bpl.push_back(0);
 
 
-    // segments of the same-level ghost fill: every element of every patch array
-    std::vector<int4> fsegs;
-    for (int i = 0; i < L->npatches; ++i)
-    {
-        const PatchDev& pd = P->patches_h[i];
-        for (int c = 0; c < P->narr; ++c)
-        {
-            const int axis = C->centering == IBAMR_SIDE ? c : -1;
-            long total = 1;
-            for (int d = 0; d < ndim; ++d) total *= pd.ihi[d] - pd.ilo[d] + 1 + 2 * P->data_gcw[d] + (d == axis ? 1 : 0);
-            for (long st = 0; st < total; st += 256)
-                fsegs.push_back(make_int4(i, c, (int)st, (int)std::min<long>(256, total - st)));
-        }
-    }
+    const std::vector<int4> fsegs = fill_segments(P);
     P->nfill_segs = (int)fsegs.size();
 
     auto cleanup_fail = [&](int code) {

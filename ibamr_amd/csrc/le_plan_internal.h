@@ -160,7 +160,7 @@ struct ibamr_plan
     int sb_off[2][2] = {};
     int* bin_patch_start_d = nullptr;  // [nmem+2]
     int* bin_patches_d = nullptr;
-    int4* fill_segs_d = nullptr;       // level ghost fill: (patch, array, first element, count) segments
+    int4* fill_segs_d = nullptr;       // level ghost fill: (patch, array, slab, first value) segments
     int nfill_segs = 0;
     void** arrays_d[MAX_SLOTS] = {};
     std::vector<void*> arrays_h[MAX_SLOTS];   // host copy of each slot's pointer table
@@ -301,6 +301,8 @@ int build_tile_lists(ibamr_plan* P);
 // le_interp.hip: per-plan interpolation set-up (dynamic LDS limits; superbin owners)
 int interp_prepare(int ndim, int kernel, int precision);
 int build_superbin_owners(ibamr_plan* P);
+// le_ghost.hip: work list of the same-level ghost fill
+std::vector<int4> fill_segments(const ibamr_plan* P);
 // le_plan.hip: timing of the main spread / interpolation launches
 int time_begin(ibamr_plan* P, int which, hipStream_t s, hipEvent_t* end);
 } // namespace ibamr
