@@ -150,280 +150,10 @@ struct SpreadArgs
     int npts;
 };
 
-template <int NDIM, int TILE>
-struct TileShape
-{
-    static constexpr int N = NDIM == 3 ? TILE * TILE * TILE : TILE * TILE;
-};
-
-template <typename T>
-struct Acc
-{
-};
-
-// Kahan-compensated add in FP32; plain add in FP64 (bitwise with the reference loop).
-__device__ __forceinline__ void acc_add(double* s, double* /*c*/, int i, double v) { s[i] = s[i] + v; }
-__device__ __forceinline__ void acc_add(float* s, float* c, int i, float v)
-{
-    const float y = v - c[i];
-    const float t = s[i] + y;
-    c[i] = (t - s[i]) - y;
-    s[i] = t;
-}
-
-template <int NDIM, int KER, typename T, int TILE>
-__global__ __launch_bounds__(WAVE) void k_spread_tiles(SpreadArgs<T> a)
-{
-    using KT = KernelTraits<KER>;
-    constexpr int W = KT::W;
-    constexpr int TN = TileShape<NDIM, TILE>::N;
-    constexpr bool FP64 = sizeof(T) == 8;
-    __shared__ T s_acc[TN];
-    __shared__ T s_cmp[FP64 ? 1 : TN];
-    __shared__ T s_w[NDIM][W][NSLOT];
-    __shared__ T s_F[NSLOT];
-    __shared__ int s_base[NDIM][NSLOT];
-    __shared__ int s_lo[NDIM][NSLOT];
-    __shared__ int s_n[NDIM][NSLOT];
-    __shared__ int s_act[NSLOT];
-
-    const int lane = threadIdx.x;
-    const TileDesc td = a.tiles[blockIdx.x];
-    if (td.patch < 0) return;  // padding of the XCD-ordered work list
-    const PatchDev P = a.patches[td.patch];
-    const int axis = a.side ? td.comp : -1;
-
-    // array box (ghosted, side box along the axis) and this tile's index range
-    int alo[3] = {0, 0, 0}, ahi[3] = {0, 0, 0}, an[3] = {1, 1, 1};
-    int flo[3] = {0, 0, 0}, fhi[3] = {0, 0, 0}, fn[3] = {1, 1, 1};
-    double xl[3] = {0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < NDIM; ++d)
-    {
-        alo[d] = P.ilo[d] - a.gcw[d];
-        ahi[d] = P.ihi[d] + a.gcw[d] + (d == axis ? 1 : 0);
-        an[d] = ahi[d] - alo[d] + 1;
-        flo[d] = alo[d] + td.t[d] * TILE;
-        fhi[d] = min(flo[d] + TILE - 1, ahi[d]);
-        if (a.mode == IBAMR_SPREAD_ACCUMULATE_INTERIOR)
-        {
-            flo[d] = max(flo[d], P.ilo[d]);
-            fhi[d] = min(fhi[d], P.ihi[d] + (d == axis ? 1 : 0));
-        }
-        fn[d] = fhi[d] - flo[d] + 1;
-        xl[d] = P.xlo[d] - (d == axis ? 0.5 * a.dx[d] : 0.0);  // LEInteractor.cpp:3689
-    }
-    if (fn[0] < 1 || fn[1] < 1 || fn[2] < 1) return;  // tile wholly in the ghost region
-    T* __restrict__ arr = a.arrays[td.patch * a.narr + (a.side ? td.comp : 0)];
-    const size_t comp_off = a.side ? 0 : (size_t)td.comp * an[0] * an[1] * (NDIM == 3 ? an[2] : 1);
-    const int fcomp = td.comp;
-    const int tcount = fn[0] * fn[1] * (NDIM == 3 ? fn[2] : 1);
-
-    // Cells whose points can reach this tile, inside the patch's Lagrangian ghost box.
-    int clo[3] = {0, 0, 0}, chi[3] = {0, 0, 0};
-    bool any = true;
-#pragma unroll
-    for (int d = 0; d < NDIM; ++d)
-    {
-        clo[d] = max(flo[d] - a.reach, P.ilo[d] - a.idx_gcw);
-        chi[d] = min(fhi[d] + a.reach, P.ihi[d] + a.idx_gcw);
-        any = any && clo[d] <= chi[d];
-    }
-    // Per-axis (bin, image offset) lists in increasing (bin, offset) order.
-    int lb[3][16], lo_[3][16], ln[3] = {0, 0, 0};
-    if (any)
-    {
-#pragma unroll
-        for (int d = 0; d < NDIM; ++d)
-        {
-            const int N = a.pshift[d];
-            const int omax = N > 0 ? 1 : 0;
-            for (int o = -omax; o <= omax; ++o)
-            {
-                const int pl = max(clo[d] - o * N, a.dom_lo[d]);
-                const int ph = min(chi[d] - o * N, a.dom_hi[d]);
-                if (pl > ph) continue;
-                const int bl = floor_div(pl - a.dom_lo[d], a.bin);
-                const int bh = floor_div(ph - a.dom_lo[d], a.bin);
-                for (int b = bl; b <= bh && ln[d] < 16; ++b)
-                {
-                    // insertion in (b, o) order
-                    int k = ln[d]++;
-                    while (k > 0 && (lb[d][k - 1] > b || (lb[d][k - 1] == b && lo_[d][k - 1] > o)))
-                    {
-                        lb[d][k] = lb[d][k - 1];
-                        lo_[d][k] = lo_[d][k - 1];
-                        --k;
-                    }
-                    lb[d][k] = b;
-                    lo_[d][k] = o;
-                }
-            }
-            any = any && ln[d] > 0;
-        }
-    }
-    if (NDIM == 2) ln[2] = 1, lb[2][0] = 0, lo_[2][0] = 0;
-
-    // Total points in the visited bins (uniform across the wavefront).
-    int total = 0;
-    if (any)
-    {
-        for (int kz = 0; kz < ln[2]; ++kz)
-            for (int ky = 0; ky < ln[1]; ++ky)
-                for (int kx = 0; kx < ln[0]; ++kx)
-                {
-                    const int b = bin_mem(NDIM, lb[0][kx], lb[1][ky], lb[2][kz], a.nb, a.nsb);
-                    total += a.bin_start[b + 1] - a.bin_start[b];
-                }
-    }
-    const bool overwrite = a.mode == IBAMR_SPREAD_OVERWRITE;
-    if (total == 0 && !overwrite) return;
-
-    // Load (accumulate: the raw LEInteractor::spread adds each contribution to
-    // the existing value, f.m4:1463) or clear (overwrite; interior mode, which
-    // spreads into zeroed data and adds the old values afterwards as
-    // LDataManager::spread does, LDataManager.cpp:594, 661-663) the tile; LDS
-    // layout is TILE-strided.
-    const bool from_old = a.mode == IBAMR_SPREAD_ACCUMULATE;
-    for (int e = lane; e < TN; e += WAVE)
-    {
-        T v = T(0);
-        const int i0 = e % TILE;
-        const int i1 = (e / TILE) % TILE;
-        const int i2 = NDIM == 3 ? e / (TILE * TILE) : 0;
-        if (from_old && i0 < fn[0] && i1 < fn[1] && i2 < fn[2])
-        {
-            const size_t g = (size_t)(flo[0] + i0 - alo[0]) +
-                             (size_t)an[0] * ((size_t)(flo[1] + i1 - alo[1]) +
-                                              (NDIM == 3 ? (size_t)an[1] * (size_t)(flo[2] + i2 - alo[2]) : 0));
-            v = arr[comp_off + g];
-        }
-        s_acc[e] = v;
-        if (!FP64) s_cmp[e] = T(0);
-    }
-    __syncthreads();
-
-    const T inv_vol = T(1.0 / a.vol);
-    for (int kz = 0; kz < ln[2] && total > 0; ++kz)
-        for (int ky = 0; ky < ln[1]; ++ky)
-            for (int kx = 0; kx < ln[0]; ++kx)
-            {
-                const int b = bin_mem(NDIM, lb[0][kx], lb[1][ky], lb[2][kz], a.nb, a.nsb);
-                const int o[3] = {lo_[0][kx], lo_[1][ky], lo_[2][kz]};
-                const int s0 = a.bin_start[b], s1 = a.bin_start[b + 1];
-                for (int base = s0; base < s1; base += NSLOT)
-                {
-                    // ---- stage up to 64 points: weights and clipped, tile-intersected ranges
-                    const int k = base + lane;
-                    int act = 0;
-                    if (k < s1)
-                    {
-                        const int4 c4 = a.cells[k];
-                        const int cc[3] = {c4.x, c4.y, c4.z};
-                        act = 1;
-#pragma unroll
-                        for (int d = 0; d < NDIM; ++d)
-                        {
-                            const int ci = cc[d] + o[d] * a.pshift[d];
-                            act = act && ci >= clo[d] && ci <= chi[d];
-                        }
-                        if (act)
-                        {
-#pragma unroll
-                            for (int d = 0; d < NDIM; ++d)
-                            {
-                                // X + Xshift with Xshift = (double)(offset) * dx  (LIndexSetData.cpp:116)
-                                const double Xu = a.X[NDIM * (size_t)k + d];
-                                const double Xs = Xu + (double)(o[d] * a.pshift[d]) * a.dx[d];
-                                T w[W];
-                                const int rel = weights_1d_u<KER>(Xs, Xu, xl[d], a.dx[d], w);
-                                const int bse = P.ilo[d] + rel;
-                                // clip to the array's ghost box (istart/istop, f.m4:1452-1457), then to the tile
-                                const int l = max(max(bse, alo[d]), flo[d]);
-                                const int h = min(min(bse + W - 1, ahi[d]), fhi[d]);
-                                act = act && l <= h;
-                                s_base[d][lane] = bse;
-                                s_lo[d][lane] = l;
-                                s_n[d][lane] = h - l + 1;
-#pragma unroll
-                                for (int j = 0; j < W; ++j) s_w[d][j][lane] = w[j];
-                            }
-                            const T Fv = a.F[(size_t)a.fdepth * k + fcomp];
-                            s_F[lane] = FP64 ? Fv : Fv * inv_vol;
-                        }
-                    }
-                    s_act[lane] = act;
-                    __syncthreads();
-                    // ---- apply the staged points one after another (single wavefront: program order)
-                    const int nst = min(NSLOT, s1 - base);
-                    for (int j = 0; j < nst; ++j)
-                    {
-                        if (!s_act[j]) continue;
-                        const int n0 = s_n[0][j], n1 = s_n[1][j];
-                        const int n2 = NDIM == 3 ? s_n[2][j] : 1;
-                        const int cnt = n0 * n1 * n2;
-                        const T Fv = s_F[j];
-                        for (int e = lane; e < cnt; e += WAVE)
-                        {
-                            const int e0 = e % n0;
-                            const int e1 = (e / n0) % n1;
-                            const int e2 = e / (n0 * n1);
-                            const int i0 = s_lo[0][j] + e0, i1 = s_lo[1][j] + e1;
-                            const T w0 = s_w[0][i0 - s_base[0][j]][j];
-                            const T w1 = s_w[1][i1 - s_base[1][j]][j];
-                            int li = (i0 - flo[0]) + TILE * (i1 - flo[1]);
-                            T c;
-                            if (NDIM == 3)
-                            {
-                                const int i2 = s_lo[2][j] + e2;
-                                const T w2 = s_w[2][i2 - s_base[2][j]][j];
-                                li += TILE * TILE * (i2 - flo[2]);
-                                if (FP64)
-                                {
-                                    const T vol = T(a.vol);
-                                    // IB: (w0*(w1*(w2/vol)))*V (f.m4:1432-1463); BS: (((w0*w1)*w2)*V)/vol (:51-64)
-                                    c = KT::IB ? (w0 * (w1 * (w2 / vol))) * Fv : (((w0 * w1) * w2) * Fv) / vol;
-                                }
-                                else
-                                    c = (w0 * (w1 * w2)) * Fv;
-                            }
-                            else
-                            {
-                                if (FP64)
-                                {
-                                    const T vol = T(a.vol);
-                                    c = KT::IB ? (w0 * (w1 / vol)) * Fv : ((w0 * w1) * Fv) / vol;
-                                }
-                                else
-                                    c = (w0 * w1) * Fv;
-                            }
-                            // remap the compact tile index to the TILE-strided LDS layout
-                            acc_add(s_acc, s_cmp, li, c);
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
-
-    // Write the tile back (strided LDS layout: TILE per row).
-    for (int e = lane; e < tcount; e += WAVE)
-    {
-        const int i0 = e % fn[0];
-        const int i1 = (e / fn[0]) % fn[1];
-        const int i2 = NDIM == 3 ? e / (fn[0] * fn[1]) : 0;
-        const int li = i0 + TILE * (i1 + TILE * i2);
-        const size_t g = (size_t)(flo[0] + i0 - alo[0]) +
-                         (size_t)an[0] * ((size_t)(flo[1] + i1 - alo[1]) +
-                                          (NDIM == 3 ? (size_t)an[1] * (size_t)(flo[2] + i2 - alo[2]) : 0));
-        T v = s_acc[li];
-        if (!FP64) v = v - s_cmp[li];
-        if (!overwrite && !from_old) v = arr[comp_off + g] + v;
-        arr[comp_off + g] = v;
-    }
-}
 } // namespace
 
 #include "le_spread3d.h"
+#include "le_spread2d.h"
 
 namespace
 {
@@ -470,7 +200,7 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
 }
 
 // Spread tile shapes built for each form; the first is the default.
-//   2-D: a 16 x 16 tile in LDS (k_spread_tiles).
+//   2-D: 16 x 16, taken as four 8 x 8 work items (k_spread2).
 //   3-D: 8 x 8 or 16 x 4 grid lines (one per lane) times a column of z values
 //     in registers (k_spread3b FP64, k_spread3 FP32C); an FP64 tile is cut along z
 //     into work items (spread_cut).  FP32C keeps two register sets per z value (the
@@ -559,7 +289,7 @@ int spread_cut(const ibamr_plan* P, const Shape& sh)
 int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
 {
     std::vector<TileDesc> tiles;
-    const Shape ext = {sh[0], sh[1], spread_cut(P, sh)};
+    const Shape ext = P->ndim == 3 ? Shape{sh[0], sh[1], spread_cut(P, sh)} : Shape{S2_TILE, S2_TILE, 1};
     out.cut = ext[2];
     const int ncomp_tiles = P->centering == IBAMR_SIDE ? P->ndim : P->depth;
     std::vector<std::vector<TileDesc>> q(8);
@@ -740,7 +470,7 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
             return fail(IBAMR_ERR_INVALID, "internal: tile shape without a kernel");
         }
         else
-            hipLaunchKernelGGL((k_spread_tiles<2, KER, T, 16>), dim3(tl.n), dim3(WAVE), 0, s, a);
+            hipLaunchKernelGGL((k_spread2<KER, T>), dim3(tl.n), dim3(64), 0, s, a);
         HIP_OK(hipGetLastError());
         if (t_end) HIP_OK(hipEventRecord(t_end, s));
         return IBAMR_OK;

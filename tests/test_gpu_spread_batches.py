@@ -3,7 +3,8 @@ bit for bit against the oracle (the order of summation does not depend on the
 batches): bins of more than 64 points beside bins of a few (batch ends inside a
 bin, never inside a 64-point chunk), every z extent of the work items (8 below
 4096 tiles, 24 from 2^17 on, 16 between), spacings whose cell volume is no power
-of two (quotients from reciprocals), tiny, zero and infinite forces."""
+of two (quotients from reciprocals), tiny, zero and infinite forces.  The same
+for the 2-D kernel (k_spread2: 8 x 8 tiles, batches of any 64 points)."""
 import numpy as np
 import pytest
 
@@ -16,9 +17,10 @@ pytestmark = pytest.mark.gpu
 
 def _check(orc, n, kernel, X, F, mode=ia.OVERWRITE):
     print("batches", n, kernel, X.shape[0], flush=True)
-    level = ia.Level.uniform_periodic(n, 3)
+    ndim = X.shape[1]
+    level = ia.Level.uniform_periodic(n, ndim)
     plan = ia.LevelPlan(level, kernel, ia.SIDE, ia.FP64, max_points=X.shape[0])
-    f = [np.zeros(ia.array_shape(level, 0, plan.data_gcw, ia.SIDE, axis=a)) for a in range(3)]
+    f = [np.zeros(ia.array_shape(level, 0, plan.data_gcw, ia.SIDE, axis=a)) for a in range(ndim)]
     dev = [_dev(a) for a in f]
     plan.bind(0, dev)
     plan.bin(_dev(X))
@@ -31,14 +33,14 @@ def _check(orc, n, kernel, X, F, mode=ia.OVERWRITE):
     plan.close()
 
 
-def _points(rng, n, dense, sparse):
+def _points(rng, n, dense, sparse, ndim=3):
     """dense points in two cells' worth of space across a bin corner and on the
     periodic edge, sparse ones anywhere."""
     h = 1.0 / n
-    X = rng.uniform(0.0, 1.0, (sparse, 3))
-    c = 8 * h * rng.integers(1, max(2, n // 8 - 1), 3)
-    D = np.remainder(c + rng.uniform(-1.2 * h, 1.2 * h, (dense, 3)), 1.0)
-    E = np.remainder(rng.uniform(-2 * h, 2 * h, (dense // 2, 3)), 1.0)
+    X = rng.uniform(0.0, 1.0, (sparse, ndim))
+    c = 8 * h * rng.integers(1, max(2, n // 8 - 1), ndim)
+    D = np.remainder(c + rng.uniform(-1.2 * h, 1.2 * h, (dense, ndim)), 1.0)
+    E = np.remainder(rng.uniform(-2 * h, 2 * h, (dense // 2, ndim)), 1.0)
     return np.concatenate([X, D, E])
 
 
@@ -48,6 +50,18 @@ def test_batches_bitwise(orc, n, kernel):
     rng = np.random.default_rng(n)
     X = _points(rng, n, 700, 5000)
     _check(orc, n, kernel, X, rng.standard_normal(X.shape))
+
+
+@pytest.mark.parametrize("n,kernel", [(24, "IB_6"), (40, "IB_4"), (37, "BSPLINE_3"), (130, "PIECEWISE_LINEAR"),
+                                      (33, "BSPLINE_5"), (48, "BSPLINE_6")])
+def test_2d_bitwise(orc, n, kernel):
+    rng = np.random.default_rng(n)
+    X = _points(rng, n, 700, 2000, 2)
+    F = rng.standard_normal(X.shape)
+    F[:20] *= 1e-200
+    F[20:30] = 0.0
+    F[30] = np.inf
+    _check(orc, n, kernel, X, F)
 
 
 def test_24_values(orc):
