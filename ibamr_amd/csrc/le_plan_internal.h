@@ -68,6 +68,13 @@ struct TileList
 };
 
 
+// One boundary operator on one component of a patch (le_ghost.hip).
+struct BdryOp
+{
+    int patch, box, kind, comp;
+    long count;  // work items
+};
+
 // radix sort and scan shapes (le_bin.hip; plan buffers are sized from them)
 constexpr int RS_BITS = 8;
 constexpr int RS_DIGITS = 1 << RS_BITS;
@@ -172,8 +179,11 @@ struct ibamr_plan
     int* pcell_off_d = nullptr;        // [npatches+1] first cell number of each patch (box order), or null
                                        // when the level has 2^31 cells or more
     int* status_d = nullptr;           // [8] redistribution counters
-    int4* bdry_patch_d = nullptr;      // physical boundary: (patch, first box, number of boxes, 0) per patch
+    char* bdry_mem_d = nullptr;        // physical boundary: the tables below, one allocation
     int* bdry_box_d = nullptr;         // [nbdry][8]: codim, location, lower[3], upper[3]
+    BdryOp* bdry_ops_d[2] = {};        // operators [forward, adjoint], in stages
+    int2* bdry_blocks_d[2] = {};       // (operator, first work item) of every workgroup, by stage
+    std::vector<int> bdry_stage_start[2];  // first workgroup of each stage, and the end
     double* bdry_coef_d = nullptr;     // Robin a, b, g over each codim-1 box's columns, per array
     long* bdry_coef_off_d = nullptr;   // [nbdry][narr] where each (box, array)'s coefficients start
     int nbdry_patches = 0;
