@@ -14,12 +14,13 @@
 //
 // The reference loops over springs, then beams, then target points, adding each
 // element's force into its nodes in element order (a scatter into F_ghost,
-// which starts at zero), and finally adds F_ghost to F.  Here every element's
-// force is computed in parallel with the reference's arithmetic, then one
-// thread per node gathers its entries from a node -> (element, role) list kept
-// in exactly that order, so every node's force is the same sequence of
-// floating-point operations as the reference loop: bitwise identical, and
-// deterministic (no atomics).
+// which starts at zero), and finally adds F_ghost to F.  Here one thread per node
+// walks a node -> (element, role) list kept in exactly that order and evaluates
+// each element's force with the reference's arithmetic where it adds it, so every
+// node's force is the same sequence of floating-point operations as the reference
+// loop: bitwise identical, and deterministic (no atomics).  An element is evaluated
+// once per node it touches (2 or 3 times): its arithmetic costs less than writing
+// its force and gathering it back.
 #include "ibamr_amd.h"
 
 #include <hip/hip_runtime.h>
@@ -76,85 +77,114 @@ __device__ inline double spring_tension(int law, const double* __restrict__ p, i
     return p[0] * (R - p[1]);
 }
 
-// Spring k: D = X_slave - X_master, R = |D|, T/R = T(R) / R, F = (T/R) D;
-// skipped when R < DBL_EPSILON (IBStandardForceGen.cpp:903-911).
-__global__ void k_spring_elem(int ns, int ndim, const int* __restrict__ m, const int* __restrict__ sl,
-                              const int* __restrict__ law, const int* __restrict__ poff,
-                              const double* __restrict__ par, const double* __restrict__ X, double* __restrict__ Fs,
-                              unsigned char* __restrict__ skip)
+struct ForceArgs
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= ns) return;
-    const int a = m[k], b = sl[k];
-    double D[3] = {0.0, 0.0, 0.0};
-    for (int d = 0; d < ndim; ++d) D[d] = X[(size_t)ndim * b + d] - X[(size_t)ndim * a + d];
-    double R2 = D[0] * D[0] + D[1] * D[1];
-    if (ndim == 3) R2 = R2 + D[2] * D[2];
-    const double R = sqrt(R2);
-    const bool sk = R < DBL_EPSILON;
-    skip[k] = sk ? 1 : 0;
-    const int o = poff[k];
-    const double T_over_R = sk ? 0.0 : spring_tension(law[k], par + o, poff[k + 1] - o, R) / R;
-    for (int d = 0; d < ndim; ++d) Fs[(size_t)ndim * k + d] = T_over_R * D[d];
-}
+    int n;
+    const int* start;
+    const int* ent;       // element << 3 | role, or pairs (role, element) when an element number needs more bits
+    int packed;
+    const int *s_m, *s_s;
+    const int *s_law, *s_off;  // null: every spring Hookean with two parameters
+    const double* s_par;
+    const int *b_m, *b_n, *b_p;
+    const double *b_K, *b_c;
+    const double *t_K, *t_E, *t_X0;
+};
 
-// Beam k: F = K (X_next + X_prev - 2 X_master - curvature) (IBStandardForceGen.cpp:1129-1131)
-__global__ void k_beam_elem(int nb, int ndim, const int* __restrict__ m, const int* __restrict__ nx,
-                            const int* __restrict__ pv, const double* __restrict__ K, const double* __restrict__ curv,
-                            const double* __restrict__ X, double* __restrict__ Fb)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nb) return;
-    const size_t im = (size_t)ndim * m[k], in = (size_t)ndim * nx[k], ip = (size_t)ndim * pv[k];
-    for (int d = 0; d < ndim; ++d)
-        Fb[(size_t)ndim * k + d] = K[k] * (((X[in + d] + X[ip + d]) - 2.0 * X[im + d]) - curv[(size_t)ndim * k + d]);
-}
-
-template <typename TF, typename TU>
-__global__ void k_node_gather(int n, int ndim, const int* __restrict__ start, const int2* __restrict__ ent,
-                              const double* __restrict__ Fs, const unsigned char* __restrict__ skip,
-                              const double* __restrict__ Fb, const int* __restrict__ t_node,
-                              const double* __restrict__ t_K, const double* __restrict__ t_E,
-                              const double* __restrict__ t_X0, const double* __restrict__ X,
-                              const TU* __restrict__ U, TF* __restrict__ F, int overwrite)
+// Bound by memory: per node of a ring with springs, beams and a target point at
+// every 4th node about 220 bytes of lists, parameters, positions and force.  1.5 M
+// nodes FP64: 85 us a call; 139 us as a spring, a beam and a gather kernel.
+template <int NDIM, typename TF, typename TU>
+__global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* __restrict__ X,
+                                                     const TU* __restrict__ U, TF* __restrict__ F, int overwrite)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (int e = start[v]; e < start[v + 1]; ++e)
+    if (v >= a.n) return;
+    double acc[NDIM], Xv[NDIM];
+#pragma unroll
+    for (int d = 0; d < NDIM; ++d)
     {
-        const int2 en = ent[e];
-        const int k = en.y;
-        switch (en.x)
+        acc[d] = 0.0;
+        Xv[d] = X[(size_t)NDIM * v + d];
+    }
+    const int e1 = a.start[v + 1];
+    for (int e = a.start[v]; e < e1; ++e)
+    {
+        int role, k;
+        if (a.packed)
         {
-        case R_SPRING_MASTER:
-            if (!skip[k])
-                for (int d = 0; d < ndim; ++d) acc[d] = acc[d] + Fs[(size_t)ndim * k + d];
-            break;
-        case R_SPRING_SLAVE:
-            if (!skip[k])
-                for (int d = 0; d < ndim; ++d) acc[d] = acc[d] - Fs[(size_t)ndim * k + d];
-            break;
-        case R_BEAM_MASTER:
-            for (int d = 0; d < ndim; ++d) acc[d] = acc[d] + 2.0 * Fb[(size_t)ndim * k + d];
-            break;
-        case R_BEAM_NEXT:
-        case R_BEAM_PREV:
-            for (int d = 0; d < ndim; ++d) acc[d] = acc[d] - Fb[(size_t)ndim * k + d];
-            break;
-        default:  // target point (IBStandardForceGen.cpp:1285-1288)
-            for (int d = 0; d < ndim; ++d)
+            const unsigned en = (unsigned)a.ent[e];
+            role = (int)(en & 7u);
+            k = (int)(en >> 3);
+        }
+        else
+        {
+            role = a.ent[2 * (size_t)e];
+            k = a.ent[2 * (size_t)e + 1];
+        }
+        if (role <= R_SPRING_SLAVE)
+        {
+            // D = X_slave - X_master, R = |D|, T/R = T(R) / R, F = (T/R) D; skipped when
+            // R < DBL_EPSILON (IBStandardForceGen.cpp:903-911)
+            const bool master = role == R_SPRING_MASTER;
+            const size_t o = (size_t)NDIM * (master ? a.s_s[k] : a.s_m[k]);
+            double D[NDIM];
+#pragma unroll
+            for (int d = 0; d < NDIM; ++d)
             {
-                const double u = U ? (double)U[(size_t)ndim * v + d] : 0.0;
-                acc[d] = acc[d] + (t_K[k] * (t_X0[(size_t)ndim * k + d] - X[(size_t)ndim * v + d]) - t_E[k] * u);
+                const double Xo = X[o + d];
+                D[d] = master ? Xo - Xv[d] : Xv[d] - Xo;
             }
-            break;
+            double R2 = D[0] * D[0] + D[1] * D[1];
+            if (NDIM == 3) R2 = R2 + D[NDIM - 1] * D[NDIM - 1];
+            const double R = sqrt(R2);
+            if (R < DBL_EPSILON) continue;
+            double T;
+            if (a.s_law)
+            {
+                const int q = a.s_off[k];
+                T = spring_tension(a.s_law[k], a.s_par + q, a.s_off[k + 1] - q, R);
+            }
+            else
+                T = spring_tension(IBAMR_SPRING_HOOKEAN, a.s_par + 2 * (size_t)k, 2, R);
+            const double T_over_R = T / R;
+#pragma unroll
+            for (int d = 0; d < NDIM; ++d)
+            {
+                const double f = T_over_R * D[d];
+                acc[d] = master ? acc[d] + f : acc[d] - f;
+            }
+        }
+        else if (role <= R_BEAM_PREV)
+        {
+            // F = K (X_next + X_prev - 2 X_master - curvature) (IBStandardForceGen.cpp:1129-1131)
+            const size_t im = (size_t)NDIM * (role == R_BEAM_MASTER ? v : a.b_m[k]),
+                         in = (size_t)NDIM * (role == R_BEAM_NEXT ? v : a.b_n[k]),
+                         ip = (size_t)NDIM * (role == R_BEAM_PREV ? v : a.b_p[k]);
+            const double K = a.b_K[k];
+#pragma unroll
+            for (int d = 0; d < NDIM; ++d)
+            {
+                const double f = K * (((X[in + d] + X[ip + d]) - 2.0 * X[im + d]) - a.b_c[(size_t)NDIM * k + d]);
+                acc[d] = role == R_BEAM_MASTER ? acc[d] + 2.0 * f : acc[d] - f;
+            }
+        }
+        else  // target point (IBStandardForceGen.cpp:1285-1288)
+        {
+            const double K = a.t_K[k], E = a.t_E[k];
+#pragma unroll
+            for (int d = 0; d < NDIM; ++d)
+            {
+                const double u = U ? (double)U[(size_t)NDIM * v + d] : 0.0;
+                acc[d] = acc[d] + (K * (a.t_X0[(size_t)NDIM * k + d] - Xv[d]) - E * u);
+            }
         }
     }
     // F += F_ghost (VecAXPY with alpha 1, :300), or F = F_ghost
-    for (int d = 0; d < ndim; ++d)
+#pragma unroll
+    for (int d = 0; d < NDIM; ++d)
     {
-        const size_t i = (size_t)ndim * v + d;
+        const size_t i = (size_t)NDIM * v + d;
         F[i] = overwrite ? (TF)acc[d] : (TF)((double)F[i] + acc[d]);
     }
 }
@@ -179,7 +209,8 @@ struct ibamr_forces
 {
     int ndim = 3, n = 0, ns = 0, nb = 0, nt = 0;
     int *s_m = nullptr, *s_s = nullptr;
-    int *s_law = nullptr, *s_off = nullptr;  // per spring: law, first parameter ([ns + 1])
+    int *s_law = nullptr, *s_off = nullptr;  // per spring: law, first parameter ([ns + 1]); null: the default
+                                             // force function for every spring, {kappa, rest} each
     double* s_par = nullptr;
     std::map<int, int> registry{{0, IBAMR_SPRING_HOOKEAN}};  // force function index -> law
     int *b_m = nullptr, *b_n = nullptr, *b_p = nullptr;
@@ -187,9 +218,8 @@ struct ibamr_forces
     int* t_i = nullptr;
     double *t_K = nullptr, *t_E = nullptr, *t_X0 = nullptr;
     int* start = nullptr;
-    int2* ent = nullptr;
-    double *Fs = nullptr, *Fb = nullptr;
-    unsigned char* skip = nullptr;
+    int* ent = nullptr;
+    bool packed = true;
 };
 
 extern "C" {
@@ -199,7 +229,7 @@ int ibamr_forces_destroy(ibamr_forces* f)
     if (!f) return IBAMR_OK;
     for (void* p : {(void*)f->s_m, (void*)f->s_s, (void*)f->s_law, (void*)f->s_off, (void*)f->s_par, (void*)f->b_m, (void*)f->b_n,
                     (void*)f->b_p, (void*)f->b_K, (void*)f->b_c, (void*)f->t_i, (void*)f->t_K, (void*)f->t_E,
-                    (void*)f->t_X0, (void*)f->start, (void*)f->ent, (void*)f->Fs, (void*)f->Fb, (void*)f->skip})
+                    (void*)f->t_X0, (void*)f->start, (void*)f->ent})
         dfree(p);
     delete f;
     return IBAMR_OK;
@@ -245,16 +275,30 @@ int ibamr_forces_create(ibamr_forces** out, int ndim, int npoints, int nsprings,
         if (bad(target_node[k])) return set_error(IBAMR_ERR_INVALID, "target point " + std::to_string(k) + ": bad node index");
         lists[target_node[k]].push_back(make_int2(R_TARGET, k));
     }
+    // an entry is one int (element << 3 | role) while the element numbers fit
+    const bool packed = std::max(nsprings, std::max(nbeams, ntargets)) <= (1 << 29);
     std::vector<int> start((size_t)npoints + 1, 0);
-    std::vector<int2> ent;
+    std::vector<int> ent;
+    size_t nent = 0;
     for (int v = 0; v < npoints; ++v)
     {
-        start[v] = (int)ent.size();
-        ent.insert(ent.end(), lists[v].begin(), lists[v].end());
+        start[v] = (int)nent;
+        for (const int2& q : lists[v])
+        {
+            if (packed)
+                ent.push_back((int)((unsigned)q.y << 3 | (unsigned)q.x));
+            else
+            {
+                ent.push_back(q.x);
+                ent.push_back(q.y);
+            }
+        }
+        nent += lists[v].size();
     }
-    start[npoints] = (int)ent.size();
+    start[npoints] = (int)nent;
 
     ibamr_forces* f = new ibamr_forces();
+    f->packed = packed;
     f->ndim = ndim;
     f->n = npoints;
     f->ns = nsprings;
@@ -268,16 +312,12 @@ int ibamr_forces_create(ibamr_forces** out, int ndim, int npoints, int nsprings,
     chk(dev_copy(&f->s_s, spring_slave, (size_t)nsprings));
     {
         // the default force function: law IBAMR_SPRING_HOOKEAN with {kappa, rest}
-        std::vector<int> law((size_t)nsprings, IBAMR_SPRING_HOOKEAN), off((size_t)nsprings + 1);
         std::vector<double> par((size_t)nsprings * 2);
-        for (int k = 0; k <= nsprings; ++k) off[k] = 2 * k;
         for (int k = 0; k < nsprings; ++k)
         {
             par[2 * (size_t)k] = spring_kappa[k];
             par[2 * (size_t)k + 1] = spring_rest[k];
         }
-        chk(dev_copy(&f->s_law, law.data(), law.size()));
-        chk(dev_copy(&f->s_off, off.data(), nsprings > 0 ? off.size() : 0));
         chk(dev_copy(&f->s_par, par.data(), par.size()));
     }
     chk(dev_copy(&f->b_m, beam_master, (size_t)nbeams));
@@ -291,14 +331,6 @@ int ibamr_forces_create(ibamr_forces** out, int ndim, int npoints, int nsprings,
     chk(dev_copy(&f->t_X0, target_X0, (size_t)ntargets * ndim));
     chk(dev_copy(&f->start, start.data(), start.size()));
     chk(dev_copy(&f->ent, ent.data(), ent.size()));
-    if (rc == IBAMR_OK && nsprings > 0)
-    {
-        if (hipMalloc(&f->Fs, sizeof(double) * (size_t)nsprings * ndim) != hipSuccess ||
-            hipMalloc(&f->skip, (size_t)nsprings) != hipSuccess)
-            rc = set_error(IBAMR_ERR_DEVICE, "hipMalloc of spring scratch failed");
-    }
-    if (rc == IBAMR_OK && nbeams > 0 && hipMalloc(&f->Fb, sizeof(double) * (size_t)nbeams * ndim) != hipSuccess)
-        rc = set_error(IBAMR_ERR_DEVICE, "hipMalloc of beam scratch failed");
     if (rc != IBAMR_OK)
     {
         ibamr_forces_destroy(f);
@@ -373,36 +405,38 @@ int ibamr_forces_compute(ibamr_forces* f, void* F, int f_precision, const double
     if (mode != IBAMR_SPREAD_ACCUMULATE && mode != IBAMR_SPREAD_OVERWRITE) return set_error(IBAMR_ERR_INVALID, "bad mode");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int B = 256;
-    if (f->ns > 0)
-    {
-        hipLaunchKernelGGL(k_spring_elem, dim3((f->ns + B - 1) / B), dim3(B), 0, s, f->ns, f->ndim, f->s_m, f->s_s,
-                           f->s_law, f->s_off, f->s_par, X, f->Fs, f->skip);
-        F_HIP(hipGetLastError());
-    }
-    if (f->nb > 0)
-    {
-        hipLaunchKernelGGL(k_beam_elem, dim3((f->nb + B - 1) / B), dim3(B), 0, s, f->nb, f->ndim, f->b_m, f->b_n,
-                           f->b_p, f->b_K, f->b_c, X, f->Fb);
-        F_HIP(hipGetLastError());
-    }
     const int ow = mode == IBAMR_SPREAD_OVERWRITE ? 1 : 0;
     const dim3 grid((f->n + B - 1) / B);
     const bool u32 = U && u_precision == IBAMR_FP32C;
-#define GATHER(TF, TU)                                                                                          \
-    hipLaunchKernelGGL((k_node_gather<TF, TU>), grid, dim3(B), 0, s, f->n, f->ndim, f->start, f->ent, f->Fs,     \
-                       f->skip, f->Fb, f->t_i, f->t_K, f->t_E, f->t_X0, X, static_cast<const TU*>(U),             \
+    const ForceArgs a{f->n,   f->start, f->ent, f->packed ? 1 : 0, f->s_m, f->s_s, f->s_law, f->s_off, f->s_par, f->b_m,
+                      f->b_n, f->b_p,   f->b_K, f->b_c,            f->t_K, f->t_E, f->t_X0};
+#define FORCES(NDIM, TF, TU)                                                                                 \
+    hipLaunchKernelGGL((k_node_forces<NDIM, TF, TU>), grid, dim3(B), 0, s, a, X, static_cast<const TU*>(U),  \
                        static_cast<TF*>(F), ow)
+#define FORCES_BY_DIM(TF, TU)          \
+    do                                 \
+    {                                  \
+        if (f->ndim == 3)              \
+            FORCES(3, TF, TU);         \
+        else                           \
+            FORCES(2, TF, TU);         \
+    } while (0)
     if (f_precision == IBAMR_FP64)
     {
-        if (u32) GATHER(double, float);
-        else GATHER(double, double);
+        if (u32)
+            FORCES_BY_DIM(double, float);
+        else
+            FORCES_BY_DIM(double, double);
     }
     else
     {
-        if (u32) GATHER(float, float);
-        else GATHER(float, double);
+        if (u32)
+            FORCES_BY_DIM(float, float);
+        else
+            FORCES_BY_DIM(float, double);
     }
-#undef GATHER
+#undef FORCES_BY_DIM
+#undef FORCES
     F_HIP(hipGetLastError());
     return IBAMR_OK;
 }
