@@ -60,170 +60,226 @@ __global__ void k_bin_keys(BinArgs a)
     a.cell[p] = make_int4(raw[0], raw[1], raw[2], 0);
 }
 
-// Exclusive scan of count[0..m) into start[0..m] (start[m] = total), three passes.
-
-__global__ __launch_bounds__(SCAN_B) void k_scan_blocks(const int* __restrict__ in, int m, int* __restrict__ out,
-                                                        int* __restrict__ bsum)
-{
-    __shared__ int s_w[SCAN_B / 64];
-    const int i = blockIdx.x * SCAN_B + threadIdx.x;
-    const int v = i < m ? in[i] : 0;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int inc = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1)
-    {
-        const int t = __shfl_up(inc, off);
-        if (lane >= off) inc += t;
-    }
-    if (lane == 63) s_w[wv] = inc;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        int run = 0;
-        for (int w = 0; w < SCAN_B / 64; ++w)
-        {
-            const int t = s_w[w];
-            s_w[w] = run;
-            run += t;
-        }
-        bsum[blockIdx.x] = run;
-    }
-    __syncthreads();
-    if (i < m) out[i] = inc - v + s_w[wv];
-}
-
-__global__ __launch_bounds__(SCAN_B) void k_scan_sums(int* __restrict__ bsum, int nb)
-{
-    // one block: exclusive scan of the block sums, SCAN_B at a time
-    __shared__ int s_w[SCAN_B / 64];
-    __shared__ int s_carry;
-    if (threadIdx.x == 0) s_carry = 0;
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int base = 0; base < nb; base += SCAN_B)
-    {
-        const int i = base + threadIdx.x;
-        const int v = i < nb ? bsum[i] : 0;
-        int inc = v;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1)
-        {
-            const int t = __shfl_up(inc, off);
-            if (lane >= off) inc += t;
-        }
-        if (lane == 63) s_w[wv] = inc;
-        __syncthreads();
-        if (threadIdx.x == 0)
-        {
-            int run = s_carry;
-            for (int w = 0; w < SCAN_B / 64; ++w)
-            {
-                const int t = s_w[w];
-                s_w[w] = run;
-                run += t;
-            }
-            s_carry = run;
-        }
-        __syncthreads();
-        if (i < nb) bsum[i] = inc - v + s_w[wv];
-        __syncthreads();
-    }
-}
-
-__global__ void k_scan_add(const int* __restrict__ part, int m, const int* __restrict__ bsum, const int* __restrict__ in,
-                           int* __restrict__ start)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const int v = part[i] + bsum[i / SCAN_B];
-    start[i] = v;
-    if (i == m - 1) start[m] = v + in[i];
-}
-
 // Stable LSD radix sort of the bin keys, carrying the point indices: after it
 // the points are grouped by bin and, inside a bin, in index order, so every
 // later kernel sees one deterministic order.  Device-wide atomics are avoided
 // (on a multi-XCD GPU they are resolved past the per-XCD L2): per pass, a
-// block histogram in LDS, one exclusive scan of the (digit, block) counts, and
-// a scatter that ranks equal digits inside a block with wave ballots.
+// block histogram in LDS, an exclusive scan of each digit's block counts, and a
+// scatter that adds up the digits' totals and ranks equal digits with wave ballots.
+//
+// At a few million keys a pass is bound by latency, not by its bytes: there are
+// only two or so workgroups per CU.  So each thread holds its keys in registers
+// (all loads in flight at once), each wavefront ranks its own run of consecutive
+// keys without a barrier, and the tile is put in digit order in LDS, so that the
+// stores of a digit's keys are consecutive.  2 M keys of
+// 20 bits: 2 x (11 + 5 + 17) us; 3 x (7 + 15 + 21) us with 8-bit digits, a scan
+// over all counts in three kernels, and a scatter of three barriers per 256 keys.
+// (Kernel by kernel an 8-bit digit is cheaper, 5 + 5 + 15 us: wide digits are taken
+// only where they save a pass.)
 
 // hist[d * nblocks + block] = number of keys of this block's tile with digit d
+template <int BITS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const int* __restrict__ keys, int n, int shift,
                                                         int nblocks, int* __restrict__ hist)
 {
-    __shared__ int s_cnt[RS_DIGITS];
+    constexpr int D = 1 << BITS;
+    __shared__ int s_cnt[D];
     const int t = threadIdx.x;
-    s_cnt[t] = 0;
-    __syncthreads();
+    for (int d = t; d < D; d += RS_THREADS) s_cnt[d] = 0;
     const int i0 = blockIdx.x * RS_TILE;
+    int key[RS_ROUNDS];
+#pragma unroll
     for (int r = 0; r < RS_ROUNDS; ++r)
     {
         const int i = i0 + r * RS_THREADS + t;
-        if (i < n) atomicAdd(&s_cnt[(keys[i] >> shift) & (RS_DIGITS - 1)], 1);  // LDS: exact, order free
+        key[r] = i < n ? keys[i] : -1;
     }
     __syncthreads();
-    hist[t * nblocks + blockIdx.x] = s_cnt[t];
+#pragma unroll
+    for (int r = 0; r < RS_ROUNDS; ++r)
+        if (key[r] >= 0) atomicAdd(&s_cnt[(key[r] >> shift) & (D - 1)], 1);  // LDS: exact, order free
+    __syncthreads();
+    for (int d = t; d < D; d += RS_THREADS) hist[(size_t)d * nblocks + blockIdx.x] = s_cnt[d];
 }
 
-// off = exclusive scan of hist (digit-major), so block b's keys of digit d go
-// to off[d * nblocks + b] onward, in tile order.  vals_in == nullptr: the
-// value of element i is i (first pass).
+__device__ __forceinline__ int wave_inclusive_sum(int v, int lane)
+{
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+    {
+        const int u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
+// off[d * nblocks + b] = keys of digit d in the blocks before b; total[d] = keys of
+// digit d.  One workgroup per digit.
+__global__ __launch_bounds__(256) void k_rs_scan(const int* __restrict__ hist, int nblocks, int* __restrict__ off,
+                                                 int* __restrict__ total)
+{
+    __shared__ int s_w[4];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const size_t row = (size_t)blockIdx.x * nblocks;
+    int run = 0;
+    for (int b0 = 0; b0 < nblocks; b0 += 256)
+    {
+        const int b = b0 + t;
+        const int v = b < nblocks ? hist[row + b] : 0;
+        const int inc = wave_inclusive_sum(v, lane);
+        if (lane == 63) s_w[wv] = inc;
+        __syncthreads();
+        int before = run, all = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+        {
+            before += w < wv ? s_w[w] : 0;
+            all += s_w[w];
+        }
+        if (b < nblocks) off[row + b] = before + inc - v;
+        run += all;
+        __syncthreads();
+    }
+    if (t == 0) total[blockIdx.x] = run;
+}
+
+// Block b's keys of digit d go to (keys of smaller digits) + off[d * nblocks + b]
+// onward, in tile order.  vals_in == nullptr: the value of element i is i (first pass).
+template <int BITS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const int* __restrict__ keys_in,
                                                            const int* __restrict__ vals_in, int n, int shift,
                                                            int nblocks, const int* __restrict__ off,
+                                                           const int* __restrict__ total,
                                                            int* __restrict__ keys_out, int* __restrict__ vals_out)
 {
-    constexpr int NW = RS_THREADS / 64;
-    __shared__ int s_run[RS_DIGITS];       // next output slot per digit
-    __shared__ int s_wc[NW][RS_DIGITS];    // per-wave count of a digit in the round, tagged with the round
+    constexpr int D = 1 << BITS;
+    constexpr int DPT = D > RS_THREADS ? D / RS_THREADS : 1;  // consecutive digits of a thread
+    __shared__ unsigned short s_wc[RS_WAVES][D];  // a wavefront's keys per digit, then where they start in the tile
+    __shared__ int s_gofs[D];                     // output position minus position in the tile
+    __shared__ int s_key[RS_TILE], s_val[RS_TILE];
+    __shared__ int s_wt[RS_WAVES], s_wl[RS_WAVES];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    s_run[t] = off[t * nblocks + blockIdx.x];
-#pragma unroll
-    for (int w = 0; w < NW; ++w) s_wc[w][t] = 0;
-    __syncthreads();
-    const unsigned long long lt = (1ull << lane) - 1ull;
     const int i0 = blockIdx.x * RS_TILE;
+    const int iw = i0 + wv * (64 * RS_ROUNDS) + lane;  // a wavefront's keys are consecutive
+    int key[RS_ROUNDS], val[RS_ROUNDS], rank[RS_ROUNDS];
+#pragma unroll
     for (int r = 0; r < RS_ROUNDS; ++r)
     {
-        const int i = i0 + r * RS_THREADS + t;
-        const bool valid = i < n;
-        const int key = valid ? keys_in[i] : 0;
-        const int val = valid ? (vals_in ? vals_in[i] : i) : 0;
-        const int dig = (key >> shift) & (RS_DIGITS - 1);
-        // lanes of this wave holding the same digit
-        unsigned long long peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < RS_BITS; ++b)
-        {
-            const unsigned long long m = __ballot((dig >> b) & 1);
-            peers &= ((dig >> b) & 1) ? m : ~m;
-        }
-        const int tag = (r + 1) << 16;
-        if (valid && (peers & lt) == 0) s_wc[wv][dig] = tag | __popcll(peers);
-        __syncthreads();
-        if (valid)
-        {
-            int pos = s_run[dig] + __popcll(peers & lt);
-            for (int w = 0; w < wv; ++w)
-            {
-                const int c = s_wc[w][dig];
-                pos += (c >> 16) == r + 1 ? (c & 0xffff) : 0;
-            }
-            keys_out[pos] = key;
-            vals_out[pos] = val;
-        }
-        __syncthreads();
-        int tot = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w)
-        {
-            const int c = s_wc[w][t];
-            tot += (c >> 16) == r + 1 ? (c & 0xffff) : 0;
-        }
-        s_run[t] += tot;
-        __syncthreads();
+        const int i = iw + r * 64;
+        key[r] = i < n ? keys_in[i] : -1;
+        val[r] = i < n ? (vals_in ? vals_in[i] : i) : 0;
     }
+    int gtot[DPT], goff[DPT];
+#pragma unroll
+    for (int k = 0; k < DPT; ++k)
+    {
+        const int d = t * DPT + k;
+        gtot[k] = d < D ? total[d] : 0;
+        goff[k] = d < D ? off[(size_t)d * nblocks + blockIdx.x] : 0;
+    }
+    for (int w = 0; w < RS_WAVES; ++w)
+        for (int d = t; d < D; d += RS_THREADS) s_wc[w][d] = 0;
+    __syncthreads();
+    // rank among the wavefront's keys of the same digit.  A wavefront's LDS operations
+    // are executed in order; volatile keeps them in order in the code.
+    {
+        volatile unsigned short* wc = s_wc[wv];
+        const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+        for (int r = 0; r < RS_ROUNDS; ++r)
+        {
+            const bool valid = key[r] >= 0;
+            const int dig = (key[r] >> shift) & (D - 1);
+            unsigned long long peers = __ballot(valid);  // lanes that hold the same digit
+#pragma unroll
+            for (int b = 0; b < BITS; ++b)
+            {
+                const unsigned long long m = __ballot((dig >> b) & 1);
+                peers &= ((dig >> b) & 1) ? m : ~m;
+            }
+            rank[r] = wc[dig] + __popcll(peers & lt);
+            if (valid && (peers & lt) == 0) wc[dig] = (unsigned short)(rank[r] + __popcll(peers));
+        }
+    }
+    __syncthreads();
+    // per digit: the wavefronts' keys in order, and the digits in order, in the tile
+    // (local) and in the output (global)
+    int cnt[DPT], lsum = 0, gsum = 0;
+#pragma unroll
+    for (int k = 0; k < DPT; ++k)
+    {
+        const int d = t * DPT + k;
+        cnt[k] = 0;
+        if (d < D)
+            for (int w = 0; w < RS_WAVES; ++w) cnt[k] += s_wc[w][d];
+        lsum += cnt[k];
+        gsum += gtot[k];
+    }
+    const int linc = wave_inclusive_sum(lsum, lane), ginc = wave_inclusive_sum(gsum, lane);
+    if (lane == 63)
+    {
+        s_wl[wv] = linc;
+        s_wt[wv] = ginc;
+    }
+    __syncthreads();
+    int lrun = linc - lsum, grun = ginc - gsum;
+#pragma unroll
+    for (int w = 0; w < RS_WAVES; ++w)
+    {
+        lrun += w < wv ? s_wl[w] : 0;
+        grun += w < wv ? s_wt[w] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < DPT; ++k)
+    {
+        const int d = t * DPT + k;
+        if (d < D)
+        {
+            s_gofs[d] = grun + goff[k] - lrun;
+            int at = lrun;
+            for (int w = 0; w < RS_WAVES; ++w)
+            {
+                const int c = s_wc[w][d];
+                s_wc[w][d] = (unsigned short)at;
+                at += c;
+            }
+        }
+        lrun += cnt[k];
+        grun += gtot[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_ROUNDS; ++r)
+        if (key[r] >= 0)
+        {
+            const int at = s_wc[wv][(key[r] >> shift) & (D - 1)] + rank[r];
+            s_key[at] = key[r];
+            s_val[at] = val[r];
+        }
+    __syncthreads();
+    const int m = min(RS_TILE, n - i0);
+#pragma unroll
+    for (int r = 0; r < RS_ROUNDS; ++r)
+    {
+        const int at = r * RS_THREADS + t;
+        if (at < m)
+        {
+            const int k = s_key[at];
+            const int pos = s_gofs[(k >> shift) & (D - 1)] + at;
+            keys_out[pos] = k;
+            vals_out[pos] = s_val[at];
+        }
+    }
+}
+
+template <int BITS>
+void radix_pass(const ibamr_plan* P, const int* kin, const int* vin, int n, int shift, int* ko, int* vo, hipStream_t s)
+{
+    const int nblk = (n + RS_TILE - 1) / RS_TILE;
+    hipLaunchKernelGGL(k_rs_hist<BITS>, dim3(nblk), dim3(RS_THREADS), 0, s, kin, n, shift, nblk, P->rs_hist_d);
+    hipLaunchKernelGGL(k_rs_scan, dim3(1 << BITS), dim3(256), 0, s, P->rs_hist_d, nblk, P->rs_off_d, P->rs_total_d);
+    hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3(nblk), dim3(RS_THREADS), 0, s, kin, vin, n, shift, nblk, P->rs_off_d,
+                       P->rs_total_d, ko, vo);
 }
 
 // start[b] = first sorted position whose key is >= b, for b in [0, m] (keys in
@@ -274,25 +330,21 @@ __global__ void k_gather_cells(const int* __restrict__ perm, const int4* __restr
 int radix_sort_pairs(const ibamr_plan* P, const int* kin, const int* vin, int n, int nbits, int* kout, int* vout,
                      int* kt, int* vt, hipStream_t s)
 {
-    const int B = 256;
-    const int passes = std::max(1, (nbits + RS_BITS - 1) / RS_BITS);
-    const int nblk = (n + RS_TILE - 1) / RS_TILE;
-    const int M = RS_DIGITS * nblk;
-    const int nsb = (M + SCAN_B - 1) / SCAN_B;
+    // As few passes as digits of RS_MAX_BITS allow, of equal digits.
+    const int passes = std::max(1, (nbits + RS_MAX_BITS - 1) / RS_MAX_BITS);
+    const int bits = (nbits + passes - 1) / passes;
+    static_assert(RS_MAX_BITS == 10, "a pass for every digit width");
     for (int p = 0; p < passes; ++p)
     {
         const bool last_parity = ((passes - 1 - p) & 1) == 0;
         int* ko = last_parity ? kout : kt;
         int* vo = last_parity ? vout : vt;
-        const int shift = p * RS_BITS;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nblk), dim3(RS_THREADS), 0, s, kin, n, shift, nblk, P->rs_hist_d);
-        hipLaunchKernelGGL(k_scan_blocks, dim3(nsb), dim3(SCAN_B), 0, s, P->rs_hist_d, M, P->scan_part_d,
-                           P->scan_tmp_d);
-        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_B), 0, s, P->scan_tmp_d, nsb);
-        hipLaunchKernelGGL(k_scan_add, dim3((M + B - 1) / B), dim3(B), 0, s, P->scan_part_d, M, P->scan_tmp_d,
-                           P->rs_hist_d, P->rs_off_d);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nblk), dim3(RS_THREADS), 0, s, kin, vin, n, shift, nblk, P->rs_off_d,
-                           ko, vo);
+        if (bits <= 8)
+            radix_pass<8>(P, kin, vin, n, p * 8, ko, vo, s);
+        else if (bits == 9)
+            radix_pass<9>(P, kin, vin, n, p * 9, ko, vo, s);
+        else
+            radix_pass<10>(P, kin, vin, n, p * 10, ko, vo, s);
         HIP_OK(hipGetLastError());
         kin = ko;
         vin = vo;

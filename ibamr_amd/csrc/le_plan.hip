@@ -201,8 +201,7 @@ int ibamr_plan_destroy(ibamr_plan* P)
     dfree(P->status_d);
     dfree(P->rs_hist_d);
     dfree(P->rs_off_d);
-    dfree(P->scan_tmp_d);
-    dfree(P->scan_part_d);
+    dfree(P->rs_total_d);
     delete P;
     return IBAMR_OK;
 }
@@ -404,7 +403,7 @@ static int plan_create_impl(ibamr_plan** out, const ibamr_level_geom* L, const i
     }
     PLAN_HIP(hipMalloc(&P->bin_start_d, sizeof(int) * (P->nmem + 2)));
     {
-        const size_t nrs = (size_t)RS_DIGITS * ((np + RS_TILE - 1) / RS_TILE);
+        const size_t nrs = ((size_t)1 << RS_MAX_BITS) * ((np + RS_TILE - 1) / RS_TILE);
         PLAN_HIP(hipMalloc(&P->keys2_d, sizeof(int) * np));
         PLAN_HIP(hipMalloc(&P->status_d, sizeof(int) * 8));
         std::vector<long long> pco(P->npatches + 1, 0);
@@ -417,13 +416,13 @@ static int plan_create_impl(ibamr_plan** out, const ibamr_level_geom* L, const i
         if (!ps && pco[P->npatches] < (1LL << 31))
         {
             std::vector<int> pci(pco.begin(), pco.end());
+            P->ncells = pci[P->npatches];
             PLAN_HIP(hipMalloc(&P->pcell_off_d, sizeof(int) * pci.size()));
             PLAN_HIP(hipMemcpy(P->pcell_off_d, pci.data(), sizeof(int) * pci.size(), hipMemcpyHostToDevice));
         }
         PLAN_HIP(hipMalloc(&P->rs_hist_d, sizeof(int) * nrs));
-        PLAN_HIP(hipMalloc(&P->rs_off_d, sizeof(int) * (nrs + 1)));
-        PLAN_HIP(hipMalloc(&P->scan_tmp_d, sizeof(int) * ((nrs + SCAN_B - 1) / SCAN_B + 1)));
-        PLAN_HIP(hipMalloc(&P->scan_part_d, sizeof(int) * nrs));
+        PLAN_HIP(hipMalloc(&P->rs_off_d, sizeof(int) * nrs));
+        PLAN_HIP(hipMalloc(&P->rs_total_d, sizeof(int) << RS_MAX_BITS));
     }
 #undef PLAN_HIP
     if (ndim == 3)

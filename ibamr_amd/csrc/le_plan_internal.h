@@ -37,7 +37,6 @@ int set_error(int code, const std::string& msg);
     } while (0)
 
 static constexpr int WAVE = 64;
-static constexpr int NSLOT = 64;
 static constexpr int MAX_SLOTS = 8;
 
 struct PatchDev
@@ -76,13 +75,12 @@ struct BdryOp
 };
 
 // radix sort and scan shapes (le_bin.hip; plan buffers are sized from them)
-constexpr int RS_BITS = 8;
-constexpr int RS_DIGITS = 1 << RS_BITS;
-constexpr int RS_THREADS = 256;            // one digit per thread in the bookkeeping
-constexpr int RS_ROUNDS = 16;              // rounds of RS_THREADS elements per block
+constexpr int RS_MAX_BITS = 10;            // widest digit of a pass
+constexpr int RS_THREADS = 512;
+constexpr int RS_WAVES = RS_THREADS / 64;
+constexpr int RS_ROUNDS = 8;               // keys per thread
 constexpr int RS_TILE = RS_THREADS * RS_ROUNDS;
-static_assert(RS_THREADS == RS_DIGITS, "one thread per digit");
-constexpr int SCAN_B = 1024;
+static_assert(RS_TILE <= 65535, "ranks inside a tile are 16-bit");
 
 
 // IndexUtilities::getCellIndex (IndexUtilities-inl.h:52-72; the level form
@@ -187,10 +185,10 @@ struct ibamr_plan
     double* bdry_coef_d = nullptr;     // Robin a, b, g over each codim-1 box's columns, per array
     long* bdry_coef_off_d = nullptr;   // [nbdry][narr] where each (box, array)'s coefficients start
     int nbdry_patches = 0;
-    int* rs_hist_d = nullptr;          // [RS_DIGITS * blocks] (digit, block) counts
-    int* rs_off_d = nullptr;           // [RS_DIGITS * blocks + 1] their exclusive scan
-    int* scan_tmp_d = nullptr;         // block sums of the scan
-    int* scan_part_d = nullptr;        // block-local exclusive prefixes of the counts
+    int* rs_hist_d = nullptr;          // [digits * blocks] (digit, block) counts
+    int* rs_off_d = nullptr;           // [digits * blocks] each digit's exclusive scan over the blocks
+    int* rs_total_d = nullptr;         // [digits] keys of each digit
+    int ncells = 0;                    // cells of all patches (pcell_off_d's last entry)
     int* perm_d = nullptr;
     int4* cell_d = nullptr;
     int4* cell_sorted_d = nullptr;
@@ -214,12 +212,6 @@ __global__ void k_fill_int(int* __restrict__ a, int n, int v)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = v;
-}
-
-__global__ void k_copy_int(const int* __restrict__ a, int n, int* __restrict__ b)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = a[i];
 }
 
 // The same permutation driven by the sorted order, for records of D positions and

@@ -23,12 +23,11 @@ struct RedistArgs
     const int* bin_patch_start;
     const int* bin_patches;
     const int* pcell_off;
-    int* key_lag;
     int* key_cell;
     int* offset;   // [n][ndim] periodic offsets, or null
-    int* blockmax; // [gridDim.x] largest Lagrangian index of each block
+    int* by_lag;   // [n] by_lag[lag[p]] = p (indices below n; lag given), see k_check_lag
     int* status;   // 0: escaped, 1: in no patch, 2: largest Lagrangian index, 3: not finite or beyond the
-                   // wrap limit, 4: negative Lagrangian index
+                   // wrap limit, 4: negative Lagrangian index, 5: indices that are no permutation of 0 .. n-1
 };
 
 constexpr int REDIST_MAX_WRAPS = 64;  // periodic wraps per coordinate before a point counts as lost
@@ -41,7 +40,6 @@ template <int NDIM>
 __global__ void k_redist_prepare(RedistArgs a)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    int lag = 0;
     if (p < a.n)
     {
         int c[3] = {0, 0, 0};
@@ -80,8 +78,8 @@ __global__ void k_redist_prepare(RedistArgs a)
                 X = fmax(X, a.xlo[d]);
                 X = fmin(X, a.xhi[d] - (a.xhi[d] - a.xlo[d]) * a.tol);
             }
-            a.X[NDIM * (size_t)p + d] = X;
-            if (a.offset) a.offset[NDIM * (size_t)p + d] = lost ? 0 : (int)round((Xr - X) / a.dx[d]);
+            if (__double_as_longlong(X) != __double_as_longlong(Xr)) a.X[NDIM * (size_t)p + d] = X;  // most stay
+            if (a.offset) a.offset[NDIM * (size_t)p + d] = lost || X == Xr ? 0 : (int)round((Xr - X) / a.dx[d]);
             // IndexUtilities::getCellIndex on the level domain
             const double v = cell_index_d(X, a.xlo[d], a.xhi[d], a.dx[d], a.dom_lo[d], a.dom_hi[d]);
             const bool inside = v >= (double)a.dom_lo[d] && v <= (double)a.dom_hi[d];
@@ -117,22 +115,15 @@ __global__ void k_redist_prepare(RedistArgs a)
             for (int d = NDIM - 1; d >= 0; --d) lin = lin * (Q.ihi[d] - Q.ilo[d] + 1) + (c[d] - Q.ilo[d]);
             cell = a.pcell_off[q] + lin;
         }
-        lag = a.lag ? a.lag[p] : p;
+        int lag = a.lag ? a.lag[p] : p;
         if (lag < 0)
         {
             atomicAdd(&a.status[4], 1);  // negative Lagrangian index
             lag = 0;
         }
         a.key_cell[p] = cell;
-        a.key_lag[p] = lag;
+        if (a.lag && lag < a.n) a.by_lag[lag] = p;
     }
-    // largest Lagrangian index of the block (no device-wide atomic: one value per block)
-    __shared__ int s_max[4];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) lag = max(lag, __shfl_xor(lag, off));
-    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = lag;
-    __syncthreads();
-    if (threadIdx.x == 0) a.blockmax[blockIdx.x] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
 }
 
 // status[2] = max of the per-block maxima (one block)
@@ -146,6 +137,30 @@ __global__ __launch_bounds__(256) void k_max_reduce(const int* __restrict__ v, i
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) *out = max(max(s_w[0], s_w[1]), max(s_w[2], s_w[3]));
+}
+
+// status[5] != 0 unless the n indices are 0 .. n-1 in some order: then by_lag holds
+// each index's only writer.  blockmax[block] = its largest index (for the sort of
+// other indices; no device-wide atomic).
+__global__ __launch_bounds__(256) void k_check_lag(const int* __restrict__ lag, const int* __restrict__ by_lag, int n,
+                                                   int* __restrict__ status, int* __restrict__ blockmax)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    bool bad = false;
+    int m = 0;
+    if (p < n)
+    {
+        const int l = lag[p];
+        bad = l < 0 || l >= n || by_lag[l] != p;
+        m = max(l, 0);
+    }
+    if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) status[5] = 1;
+    __shared__ int s_max[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) blockmax[blockIdx.x] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
 }
 
 __global__ void k_gather_int(const int* __restrict__ src, const int* __restrict__ idx, int n, int* __restrict__ dst)
@@ -226,20 +241,21 @@ int ibamr_plan_redistribute(ibamr_plan* P, double* X, const int* lag_index, int 
     a.bin_patch_start = P->bin_patch_start_d;
     a.bin_patches = P->bin_patches_d;
     a.pcell_off = P->pcell_off_d;
-    a.key_lag = P->keys_d;
-    a.key_cell = reinterpret_cast<int*>(P->cell_d);  // cell_d holds 4 ints per point; the binning is void now
+    // gathered into keys_d by Lagrangian index below; cell_d holds 4 ints per point (the binning is void now)
+    a.key_cell = lag_index ? reinterpret_cast<int*>(P->cell_d) : P->keys_d;
+    a.by_lag = P->perm_d;
     a.offset = periodic_offset;
     a.status = P->status_d;
-    a.blockmax = P->rs_hist_d;  // free until the sorts below; holds >= max_points / 16 ints
     if (npoints > 0)
     {
-        static_assert(RS_TILE / RS_DIGITS <= 256, "block maxima must fit the histogram buffer");
         const int G = (npoints + B - 1) / B;
         if (P->ndim == 3)
             hipLaunchKernelGGL(k_redist_prepare<3>, dim3(G), dim3(B), 0, s, a);
         else
             hipLaunchKernelGGL(k_redist_prepare<2>, dim3(G), dim3(B), 0, s, a);
-        hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(256), 0, s, P->rs_hist_d, G, P->status_d + 2);
+        if (lag_index)  // rs_hist_d: free until the sorts below; holds >= max_points / 4 ints
+            hipLaunchKernelGGL(k_check_lag, dim3(G), dim3(B), 0, s, lag_index, P->perm_d, npoints, P->status_d,
+                               P->rs_hist_d);
         HIP_OK(hipGetLastError());
     }
     int st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -256,28 +272,29 @@ int ibamr_plan_redistribute(ibamr_plan* P, double* X, const int* lag_index, int 
         return fail(IBAMR_ERR_OUT_OF_DOMAIN, std::to_string(st[1]) + " point(s) lie in no patch of the level");
     if (npoints > 0)
     {
-        int* key_cell = reinterpret_cast<int*>(P->cell_d);
         const int G = (npoints + B - 1) / B;
-        const int* order1 = nullptr;
+        const int* order1 = nullptr;  // no indices given: position = index
         if (lag_index)
         {
             // by Lagrangian index first, then (stable) by cell: patches in level order, cells in box order,
-            // nodes of a cell by Lagrangian index (LDataManager.cpp:1498-1503, 2897-2908)
-            int rc = radix_sort_pairs(P, P->keys_d, nullptr, npoints, bits_for(st[2]), P->keys_sorted_d, P->perm_d,
-                                      P->keys2_d, P->idx_d, s);
-            if (rc != IBAMR_OK) return rc;
-            hipLaunchKernelGGL(k_gather_int, dim3(G), dim3(B), 0, s, key_cell, P->perm_d, npoints, P->keys_d);
+            // nodes of a cell by Lagrangian index (LDataManager.cpp:1498-1503, 2897-2908).
+            // Indices that are 0 .. n-1 in some order (all points of a level on this
+            // GPU) are in order in perm_d already (2 M points: two passes over them
+            // instead of three of a sort); others are sorted.
+            if (st[5] != 0)
+            {
+                hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(256), 0, s, P->rs_hist_d, G, P->status_d + 2);
+                HIP_OK(hipMemcpyAsync(st, P->status_d, sizeof(st), hipMemcpyDeviceToHost, s));
+                HIP_OK(hipStreamSynchronize(s));
+                const int rc = radix_sort_pairs(P, lag_index, nullptr, npoints, bits_for(st[2]), P->keys_sorted_d,
+                                                P->perm_d, P->keys2_d, P->idx_d, s);
+                if (rc != IBAMR_OK) return rc;
+            }
+            hipLaunchKernelGGL(k_gather_int, dim3(G), dim3(B), 0, s, a.key_cell, P->perm_d, npoints,
+                               P->keys_d);
             order1 = P->perm_d;
         }
-        else
-        {
-            // Lagrangian index = position: already in index order
-            hipLaunchKernelGGL(k_copy_int, dim3(G), dim3(B), 0, s, key_cell, npoints, P->keys_d);
-        }
-        int total = 0;
-        HIP_OK(hipMemcpyAsync(&total, P->pcell_off_d + P->npatches, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIP_OK(hipStreamSynchronize(s));
-        const int rc = radix_sort_pairs(P, P->keys_d, order1, npoints, bits_for(std::max(0, total - 1)),
+        const int rc = radix_sort_pairs(P, P->keys_d, order1, npoints, bits_for(std::max(0, P->ncells - 1)),
                                         P->keys_sorted_d, new_order, P->keys2_d, P->idx_d, s);
         if (rc != IBAMR_OK) return rc;
     }
