@@ -350,7 +350,7 @@ int ibamr_plan_interp(ibamr_plan* P, int slot, void* U, const double* X, void* s
         hipEvent_t t_end = nullptr;
         if (NDIM == 3)
         {
-            // one workgroup per superbin; LDS holds one staged block of the array
+            // one workgroup per superbin (or half of one); LDS holds one staged block of the array
             // (the kernel's dynamic LDS limit is raised once, at plan creation)
             const int elems = interp3_lds_elems<KER, T>();
             const int bytes = elems * (int)sizeof(T);
@@ -358,20 +358,21 @@ int ibamr_plan_interp(ibamr_plan* P, int slot, void* U, const double* X, void* s
             if (trc != IBAMR_OK) return trc;
             const int nsb = P->nsb[0] * P->nsb[1] * P->nsb[2];
             const int nrow = P->nsb[1] * P->nsb[2];
-            const int per = (nrow + 7) / 8 * P->nsb[0];  // superbins per XCD (see k_interp3)
+            constexpr int zs = interp3_zs<KER, T>();
+            const int per = ((nrow + 7) / 8 * P->nsb[0]) << zs;  // workgroups per XCD (see k_interp3)
             if constexpr (sizeof(T) == 4)
             {
                 if (a.st)  // the spread set-up's stencils of these positions
                 {
                     hipLaunchKernelGGL((k_interp3<KER, T, true>), dim3(8 * per), dim3(I3_THREADS), bytes, s, a,
-                                       elems, nsb, P->nsb[0]);
+                                       elems, nsb, P->nsb[0], zs);
                     HIP_OK(hipGetLastError());
                     if (t_end) HIP_OK(hipEventRecord(t_end, s));
                     return IBAMR_OK;
                 }
             }
             hipLaunchKernelGGL((k_interp3<KER, T, false>), dim3(8 * per), dim3(I3_THREADS), bytes, s, a, elems, nsb,
-                               P->nsb[0]);
+                               P->nsb[0], zs);
         }
         else
         {

@@ -2,7 +2,7 @@
 // le_interp.hip, which defines InterpArgs and Sum).
 //
 // Interpolation (k_interp3): one IBAMR_I3_THREADS-thread (512) workgroup per
-// superbin (2x2x2 bins = 16^3 cells).  For each array it finds the exact stencil extent of its
+// superbin (2x2x2 bins = 16^3 cells) or half of one (interp3_zs).  For each array it finds the exact stencil extent of its
 // points, stages that block of the ghosted array into LDS with coalesced
 // loads, then each thread sums the W^3 stencil of its points from LDS.
 #pragma once
@@ -24,10 +24,26 @@ constexpr int interp3_edge()
     return 16 + KernelTraits<KER>::W;
 }
 
+// 1: a workgroup takes the lower or the upper half of a superbin (16 x 16 x 8 cells).
+// While a workgroup waits for its block or sums from it, another one on the CU can do
+// the other, if the LDS holds both: with 22^3 doubles (IB_6) it does not, with halves
+// it does, for 1.27 times the halo.  Halves against whole superbins: IB_6 FP64, 8.4 M
+// points on 512^3: 4325 / 4672 us; IB_4 FP64, 1 M points on 256^3: 160 / 168 us, 0.5 M
+// on 200^3: 83 / 93 us.  Not where the halo is all that changes: FP32C (three or four
+// blocks fit as they are) IB_6 512^3 1832 / 1394 us, IB_4 and BSPLINE_3 of a 384^3
+// level 231 / 217 and 169 / 164 us (but 42 / 58 us for BSPLINE_3, 0.5 M on 200^3);
+// PIECEWISE_LINEAR FP64, 300^3: 411 / 311 us (little to sum per staged value).
+template <int KER, typename T>
+constexpr int interp3_zs()
+{
+    return KER != K_PWL && sizeof(T) == 8 ? 1 : 0;
+}
+
+// A cut superbin's block has 8 cells less along z.
 template <int KER, typename T>
 constexpr int interp3_lds_elems()
 {
-    return interp3_edge<KER>() * interp3_edge<KER>() * interp3_edge<KER>();
+    return interp3_edge<KER>() * interp3_edge<KER>() * (interp3_edge<KER>() - 8 * interp3_zs<KER, T>());
 }
 
 // Owning patch of a sorted point: the patch whose selection box holds its
@@ -55,7 +71,7 @@ __device__ __forceinline__ int interp_owner(const InterpArgs<T>& a, int k, const
 }
 
 template <int KER, typename T, bool LD>
-__global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds_elems, int nsb, int nsx)
+__global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds_elems, int nsb, int nsx, int zs)
 {
     using KT = KernelTraits<KER>;
     constexpr int W = KT::W;
@@ -78,9 +94,11 @@ __global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds
     // rows in order: a row's superbins share their x halo in one L2, and every
     // XCD gets a share of every region of the point cloud.
     const int xi = (int)(blockIdx.x % 8), qi = (int)(blockIdx.x / 8);
-    const int sb = (xi + 8 * (qi / nsx)) * nsx + qi % nsx;
+    const int nqx = nsx << zs, qx = qi % nqx;
+    const int sb = (xi + 8 * (qi / nqx)) * nsx + (qx >> zs);
     if (sb >= nsb) return;
-    const int s0 = a.bin_start[sb * 8], s1 = a.bin_start[sb * 8 + 8];
+    const int part = qx & zs;  // zs = 1: the lower or the upper four bins
+    const int s0 = a.bin_start[sb * 8 + 4 * part], s1 = a.bin_start[sb * 8 + (zs ? 4 * part + 4 : 8)];
     if (s0 == s1) return;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wv = tid >> 6;
@@ -94,7 +112,8 @@ __global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds
         {
             const int v = tid / 3, d = tid % 3;
             const int sc = d == 0 ? sb % nsx : (d == 1 ? (sb / nsx) % a.nsy : sb / nsx / a.nsy);
-            const int clo = a.lev_lo[d] + a.sbc * sc, chi = min(clo + a.sbc - 1, a.dom_hi[d]);
+            const int cut = d == 2 ? zs : 0, nc = a.sbc >> cut;
+            const int clo = a.lev_lo[d] + a.sbc * sc + (cut ? nc * part : 0), chi = min(clo + nc - 1, a.dom_hi[d]);
             s_lo[v][d] = clo + a.sb_off[v][0];
             s_hi[v][d] = chi + a.sb_off[v][1];
         }
@@ -301,8 +320,8 @@ __global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds
                 {
                     if (!PRE)
                     {
-                        const double xl = Pq.xlo[d] - (d == axis ? 0.5 * a.dx[d] : 0.0);
-                        bse[d] = Pq.ilo[d] + weights_1d<KER>(a.X[3 * (size_t)k + d], xl, a.dx[d], w[d]);
+                        const double X = a.X[3 * (size_t)k + d], xl = Pq.xlo[d] - (d == axis ? 0.5 * a.dx[d] : 0.0);
+                        bse[d] = Pq.ilo[d] + weights_1d<KER>(X, xl, a.dx[d], w[d]);
                     }
                     else if (pre_ld)
                     {
