@@ -11,15 +11,15 @@
 //    stable LSD radix sort of the points by spread bin (a cube of cells; no
 //    device-wide atomics); CSR offsets by a binary search per bin.
 //  * spread: owner-computes gather.  A tile of grid values of one array (side
-//    axis or depth component) of one patch belongs to one wavefront (2-D here:
-//    a 16x16 tile in LDS; 3-D in le_kernels3d.h: 8x8 columns of z values in
-//    registers).  It visits the bins whose points can reach the tile in a fixed
+//    axis or depth component) of one patch belongs to one workgroup (2-D in
+//    le_spread2d.h: one value per lane; 3-D in le_spread3d.h: one wavefront, 8x8
+//    columns of z values in registers).  It visits the bins whose points can reach the tile in a fixed
 //    order (bin z, image z, bin y, image y, bin x, image x) and the points of
 //    each bin in index order, so every grid value sums its contributions in a
 //    fixed order: no atomics, bitwise reproducible.  Periodic images
 //    (LIndexSetData.cpp:80-117) are generated on the fly from the bin offsets.
 //  * interp: 2-D one thread per point in bin order; 3-D one workgroup per
-//    superbin with the grid block staged in LDS (le_kernels3d.h).
+//    superbin with the grid block staged in LDS (le_interp3d.h).
 //  * around the path: redistribution at a regrid (radix sorts by patch, cell and
 //    Lagrangian index), same-level and periodic ghost fills, the physical
 //    boundary (Robin) operators, the forward-Euler update.

@@ -422,13 +422,11 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
         const TileList& tl = P->tlists[P->tcur];
         if constexpr (NDIM == 3)
         {
-            // FP32C packs chunks across bins; FP64 cuts them per bin (the oracle's fixed order)
-            constexpr bool MERGE = sizeof(T) == 4;
             const dim3 G(tl.n), B(64);
 #define IBAMR_S3(TX, ZC)                                                              \
     if (tl.shape[0] == TX && tl.shape[2] == ZC)                                       \
     {                                                                                 \
-        hipLaunchKernelGGL((k_spread3<KER, T, MERGE, ZC, TX>), G, B, 0, s, a);        \
+        hipLaunchKernelGGL((k_spread3<KER, ZC, TX>), G, B, 0, s, a);                  \
         HIP_OK(hipGetLastError());                                                    \
         if (t_end) HIP_OK(hipEventRecord(t_end, s));                                  \
         return IBAMR_OK;                                                              \

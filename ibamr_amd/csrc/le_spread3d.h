@@ -1,26 +1,21 @@
 // le_spread3d.h -- 3-D spread kernel for gfx950 (included by le_spread.hip,
 // which defines SpreadArgs, PatchDev and TileDesc).
 //
-// Spread (k_spread3): owner-computes, register-resident.  One wavefront owns a
+// FP32C spread (k_spread3): owner-computes, register-resident.  One wavefront owns a
 // column tile of one array: TX x TY (x, y) grid lines (8 x 8 or 16 x 4), one
 // per lane, times ZC consecutive z values held in registers.  Points that can reach the
-// tile are staged 64 at a time: each lane takes one point's stencil (FP64
-// computes the reference's weights; FP32C loads the starts and weights the
-// set-up pass computed once per point) and writes the x and y weights, aligned
-// to the tile's lanes and zero-padded, plus the z weights to LDS.  The staged
+// tile are staged 64 at a time: each lane takes one point's stencil (the starts and
+// weights that the set-up pass computed once per point) and writes the x and y weights,
+// aligned to the tile's lanes and zero-padded, plus the z weights to LDS.  The staged
 // points are then applied grouped by their first z index: a ballot per z start
 // yields the points with that start, so every register index is a compile-time
 // constant (no dynamic VGPR indexing).  Per point and lane the work is two LDS
 // reads, one product and W fused multiply-adds.  No atomics: each grid value
 // lives in one lane's register and receives its contributions in a fixed
-// order, so results are bitwise reproducible.
-//   FP32C: each chunk's contributions go to FP32 partial sums, which are
-//          folded into FP64 totals after the chunk (a chunk holds at most 64
-//          points, so the FP32 sums stay short).
-//   FP64:  the reference operation order per contribution
-//          (IB: (w0*(w1*(w2/vol)))*F, BSPLINE: (((w0*w1)*w2)*F)/vol) and
-//          sequential adds, over chunks cut per bin, so the result equals the
-//          reference loop run over the oracle's z-bucketed entry order.
+// order, so results are bitwise reproducible.  Each chunk's contributions go to FP32
+// partial sums, which are folded into FP64 totals after the chunk (a chunk holds at
+// most 64 points, so the FP32 sums stay short).
+// FP64 (k_spread3b) and FP32C columns swept along z (k_spread3s): see there.
 #pragma once
 
 namespace
@@ -54,24 +49,21 @@ __device__ __forceinline__ double uniform_double(double v)
     return __hiloint2double(hi, lo);
 }
 
-template <int KER, typename T, bool MERGE, int ZC, int TX>
-__global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
+template <int KER, int ZC, int TX>
+__global__ __launch_bounds__(64) void k_spread3(SpreadArgs<float> a)
 {
+    using T = float;
     using KT = KernelTraits<KER>;
     constexpr int W = KT::W;
-    constexpr bool FP64 = sizeof(T) == 8;
-    // FP32C stages the set-up pass's stencils, except for kernels whose
-    // stencil side depends on the unshifted X (an image's differs)
-    constexpr bool PRECOMP = !FP64 && !side_by_unshifted_x<KER>();
+    // the set-up pass's stencils are staged, except for kernels whose stencil side
+    // depends on the unshifted X (an image's differs)
+    constexpr bool PRECOMP = !side_by_unshifted_x<KER>();
     constexpr int TY = 64 / TX;  // the 64 lanes: TX x TY grid lines
     constexpr int PX = s3_pad<TX>(), PY = s3_pad<TY>();
     static_assert(TX * TY == 64, "one lane per grid line");
     __shared__ T s_rx[64 * PX];
     __shared__ T s_ry[64 * PY];
     __shared__ T s_wz[64 * 8];
-    __shared__ T s_F[64];
-    __shared__ int s_dx0[64];
-    __shared__ int s_dy0[64];
     __shared__ int s_lb[3][16];
     __shared__ int s_lo[3][16];
     __shared__ int s_ln[3];
@@ -159,16 +151,15 @@ __global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
     const int nx = s_ln[0], ny = s_ln[1], nz = s_ln[2];
     const int ncomb = nx * ny * nz;
 
-    // registers: tile values, accumulated in FP64 (FP32C: plus the chunk's
-    // FP32 partial sums)
+    // registers: tile values, accumulated in FP64, plus the chunk's FP32 partial sums
     double acc[ZC];
-    T part[FP64 ? 1 : ZC];
+    T part[ZC];
     const bool overwrite = a.mode == IBAMR_SPREAD_OVERWRITE;
 #pragma unroll
     for (int z = 0; z < ZC; ++z)
     {
         acc[z] = 0.0;
-        if (!FP64) part[z] = T(0);
+        part[z] = T(0);
     }
 
     // total number of points in the visited bins; an empty tile keeps its values.
@@ -203,7 +194,6 @@ __global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
     }
 
     const T inv_vol = T(1.0 / a.vol);
-    const T vol = T(a.vol);
     for (int cb = 0; cb < ncomb && total > 0; cb += S3_MAXCOMB)
     {
         // ---- this group of combinations: ranges and their prefix (in canonical order)
@@ -239,55 +229,37 @@ __global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
         const int ngc = min(S3_MAXCOMB, ncomb - cb);
         const int gtotal = s_cp[ngc];
 
-        // chunks: MERGE packs any 64 consecutive points of the group; otherwise a
-        // chunk never crosses a combination (64-point blocks of each bin).  The
-        // next chunk's point data is loaded while the current one is applied.
-        int cq = 0, cr = 0, crp = 0;
-        auto normalize = [&]() {
-            if (!MERGE)
-                while (cr < ngc && crp >= s_cl[cr])
-                {
-                    ++cr;
-                    crp = 0;
-                }
-        };
+        // chunks: any 64 consecutive points of the group.  The next chunk's point
+        // data is loaded while the current one is applied.
+        int cq = 0;
         auto lane_point = [&](int& k, int& oc) {
             k = -1;
             oc = 13;
-            if (MERGE)
+            const int q = cq + lane;
+            if (q < gtotal)
             {
-                const int q = cq + lane;
-                if (q < gtotal)
+                int lo = 0, hi = ngc - 1;  // last combination with prefix <= q
+                while (lo < hi)
                 {
-                    int lo = 0, hi = ngc - 1;  // last combination with prefix <= q
-                    while (lo < hi)
-                    {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (s_cp[mid] <= q)
-                            lo = mid;
-                        else
-                            hi = mid - 1;
-                    }
-                    k = s_cs[lo] + (q - s_cp[lo]);
-                    oc = s_co[lo];
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_cp[mid] <= q)
+                        lo = mid;
+                    else
+                        hi = mid - 1;
                 }
-            }
-            else if (cr < ngc && crp + lane < s_cl[cr])
-            {
-                k = s_cs[cr] + crp + lane;
-                oc = s_co[cr];
+                k = s_cs[lo] + (q - s_cp[lo]);
+                oc = s_co[lo];
             }
         };
-        normalize();
-        bool cvalid = MERGE ? cq < gtotal : cr < ngc;
+        bool cvalid = cq < gtotal;
         int nk, noc;
         int4 nc4 = make_int4(0, 0, 0, 0);
         double nX[3] = {0.0, 0.0, 0.0};
         T nF = T(0);
-        int nst[3] = {0, 0, 0};   // FP32C: precomputed stencil starts and weights
+        int nst[3] = {0, 0, 0};   // precomputed stencil starts and weights
         float nw[3][W];
-        // the lane's point of the current chunk: position (FP64) or precomputed
-        // starts and weights (FP32C, rows of the point's axis variants), F, cell
+        // the lane's point of the current chunk: precomputed starts and weights (rows
+        // of the point's axis variants) or position, F, cell
         auto load_point = [&]() {
             if (nk < 0) return;
             nc4 = a.cells[nk];
@@ -366,33 +338,22 @@ __global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
                         for (int i = 0; i < TX; ++i) rx[i] = T(0);
 #pragma unroll
                         for (int i = 0; i < TY; ++i) ry[i] = T(0);
-                        const T fx = FP64 ? T(1) : (KT::IB ? Fv : Fv * inv_vol);
+                        const T fx = KT::IB ? Fv : Fv * inv_vol;
 #pragma unroll
                         for (int j = 0; j < W; ++j)
                         {
-                            if ((unsigned)(dx0 + j) < (unsigned)TX) rx[dx0 + j] = FP64 ? w[0][j] : w[0][j] * fx;
+                            if ((unsigned)(dx0 + j) < (unsigned)TX) rx[dx0 + j] = w[0][j] * fx;
                             if ((unsigned)(dy0 + j) < (unsigned)TY) ry[dy0 + j] = w[1][j];
-                            // FP64 IB folds 1/vol into w2 exactly as the reference (f.m4:1435)
-                            s_wz[lane * 8 + j] = (FP64 && KT::IB) ? w[2][j] / vol
-                                                                  : ((!FP64 && KT::IB) ? w[2][j] * inv_vol : w[2][j]);
+                            s_wz[lane * 8 + j] = KT::IB ? w[2][j] * inv_vol : w[2][j];
                         }
-                        s_F[lane] = Fv;
-                        s_dx0[lane] = dx0;
-                        s_dy0[lane] = dy0;
                         my_zz = zz;
                     }
                 }
             }
             __syncthreads();
             // advance, and load the next chunk's points while this one is applied
-            if (MERGE)
-                cq += 64;
-            else
-            {
-                crp += 64;
-                normalize();
-            }
-            cvalid = MERGE ? cq < gtotal : cr < ngc;
+            cq += 64;
+            cvalid = cq < gtotal;
             nk = -1;
             if (cvalid) lane_point(nk, noc);
             load_point();
@@ -422,55 +383,20 @@ __global__ __launch_bounds__(64) void k_spread3(SpreadArgs<T> a)
                             wz[i] = s_wz[j * 8 + i];
                             wz2[i] = s_wz[j2 * 8 + i];
                         }
-                        if (!FP64)
-                        {
-                            const T b = wx * wy;
-                            const T b2 = two ? wx2 * wy2 : T(0);
+                        const T b = wx * wy;
+                        const T b2 = two ? wx2 * wy2 : T(0);
 #pragma unroll
-                            for (int i = 0; i < W; ++i)
-                                if (zz + i >= 0 && zz + i < ZC)
-                                    part[zz + i] = fmaf(b2, wz2[i], fmaf(b, wz[i], part[zz + i]));
-                        }
-                        else
-                        {
-                            const bool inside = (unsigned)(x - s_dx0[j]) < (unsigned)W &&
-                                                (unsigned)(y - s_dy0[j]) < (unsigned)W;
-                            const bool inside2 = two && (unsigned)(x - s_dx0[j2]) < (unsigned)W &&
-                                                 (unsigned)(y - s_dy0[j2]) < (unsigned)W;
-                            const T Fj = s_F[j], Fj2 = s_F[j2];
-                            if (inside)
-                            {
-#pragma unroll
-                                for (int i = 0; i < W; ++i)
-                                    if (zz + i >= 0 && zz + i < ZC)
-                                    {
-                                        const T c = KT::IB ? (wx * (wy * wz[i])) * Fj : (((wx * wy) * wz[i]) * Fj) / vol;
-                                        acc[zz + i] = acc[zz + i] + c;
-                                    }
-                            }
-                            if (inside2)
-                            {
-#pragma unroll
-                                for (int i = 0; i < W; ++i)
-                                    if (zz + i >= 0 && zz + i < ZC)
-                                    {
-                                        const T c = KT::IB ? (wx2 * (wy2 * wz2[i])) * Fj2
-                                                           : (((wx2 * wy2) * wz2[i]) * Fj2) / vol;
-                                        acc[zz + i] = acc[zz + i] + c;
-                                    }
-                            }
-                        }
+                        for (int i = 0; i < W; ++i)
+                            if (zz + i >= 0 && zz + i < ZC)
+                                part[zz + i] = fmaf(b2, wz2[i], fmaf(b, wz[i], part[zz + i]));
                     }
                 }
-                if (!FP64)
-                {
-                    // fold the chunk's partial sums into the FP64 totals
+                // fold the chunk's partial sums into the FP64 totals
 #pragma unroll
-                    for (int z = 0; z < ZC; ++z)
-                    {
-                        acc[z] = acc[z] + (double)part[z];
-                        part[z] = T(0);
-                    }
+                for (int z = 0; z < ZC; ++z)
+                {
+                    acc[z] = acc[z] + (double)part[z];
+                    part[z] = T(0);
                 }
             }
             __syncthreads();
