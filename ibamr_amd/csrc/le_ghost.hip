@@ -410,11 +410,16 @@ __host__ __device__ inline void bd_edge(int loc, int* e, int* n1, int* n2, int* 
     }
 }
 
+// layers from an edge or corner box's normal face b inward to the mirror image of
+// its outermost layer: the box's extent, more if it does not touch the patch
+__host__ __device__ inline int bd_inward(int up, int b, int lo, int hi) { return up ? hi - b : b - lo; }
+
 // cell data, 3-D edges.  Forward: work item = ghost value (all read values lie
-// outside the edge box).  Adjoint: work item = target at one edge index: a value of
-// the mirror square (targets m, and on its sides those of xc, xd), a ghost value
-// beside face 1 (xb) or beside face 2 (xa); it walks the sources in the reference's
-// order (c2, then c1) and takes the updates that name it.
+// outside the edge box).  Adjoint: work item = possible target at one edge index: a
+// value of the square from (b1, b2) inward to the mirror image (targets m, and on its
+// sides those of the subtractions), a ghost value beside face 1 or beside face 2; it
+// walks the sources in the reference's order (c2, then c1) and takes the updates that
+// name it (none in the gap that a box off the patch leaves in the square).
 template <typename T>
 __device__ void bd_cc_edge(const BPatch<T>& P, int comp, int loc, const int* flo, const int* fhi, int adjoint, long t)
 {
@@ -441,13 +446,14 @@ __device__ void bd_cc_edge(const BPatch<T>& P, int comp, int loc, const int* flo
         *val(c1, c2) = (T)v;
         return;
     }
+    const int q1 = bd_inward(u1, b1, flo[n1], fhi[n1]), q2 = bd_inward(u2, b2, flo[n2], fhi[n2]);
     int t1, t2;  // the target
-    if (r < k1 * k2)
-        t1 = mir1(flo[n1] + r % k1), t2 = mir2(flo[n2] + r / k1);
-    else if (r < k1 * k2 + k1)
-        t1 = flo[n1] + (r - k1 * k2), t2 = b2;
+    if (r < q1 * q2)
+        t1 = b1 - s1 * (r % q1), t2 = b2 - s2 * (r / q1);
+    else if (r < q1 * q2 + k1)
+        t1 = flo[n1] + (r - q1 * q2), t2 = b2;
     else
-        t1 = b1, t2 = flo[n2] + (r - k1 * k2 - k1);
+        t1 = b1, t2 = flo[n2] + (r - q1 * q2 - k1);
     T v = *val(t1, t2);
     for (int c2 = flo[n2]; c2 <= fhi[n2]; ++c2)
         for (int c1 = flo[n1]; c1 <= fhi[n1]; ++c1)
@@ -464,12 +470,13 @@ __device__ void bd_cc_edge(const BPatch<T>& P, int comp, int loc, const int* flo
 }
 
 // cell data, corners (codim == ndim): as the edges, the sources in (z, y, x) order;
-// targets: the mirror cube, and the ghost values along axis d beside the corner cell
+// targets: the cube from b inward to the mirror image, and the ghost values along
+// axis d beside the corner cell
 template <typename T>
 __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* flo, const int* fhi, int adjoint, long t)
 {
     const int nd = P.ndim;
-    int b[3] = {0, 0, 0}, s[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, n[3] = {1, 1, 1};
+    int b[3] = {0, 0, 0}, s[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, n[3] = {1, 1, 1}, in[3] = {1, 1, 1};
     for (int d = 0; d < nd; ++d)
     {
         const int up = (loc >> d) & 1;
@@ -477,8 +484,9 @@ __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* f
         s[d] = up ? 1 : -1;
         lo[d] = flo[d];
         n[d] = fhi[d] - flo[d] + 1;
+        in[d] = bd_inward(up, b[d], flo[d], fhi[d]);
     }
-    const int cube = n[0] * n[1] * n[2];
+    const int cube = in[0] * in[1] * in[2];
     auto source = [&](int q, int* x, int* m) {
         x[0] = lo[0] + q % n[0], x[1] = lo[1] + (q / n[0]) % n[1], x[2] = lo[2] + q / (n[0] * n[1]);
         m[2] = 0;
@@ -507,8 +515,12 @@ __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* f
     int y[3] = {b[0], b[1], b[2]};
     if (t < cube)
     {
-        source((int)t, x, m);
-        for (int d = 0; d < nd; ++d) y[d] = m[d];
+        int r = (int)t;
+        for (int d = 0; d < nd; ++d)
+        {
+            y[d] = b[d] - s[d] * (r % in[d]);
+            r /= in[d];
+        }
     }
     else
     {
@@ -518,7 +530,7 @@ __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* f
     }
     T* target = P.at(0, comp, y);
     T v = *target;
-    for (int q = 0; q < cube; ++q)
+    for (int q = 0; q < n[0] * n[1] * n[2]; ++q)
     {
         source(q, x, m);
         const double Ug = (double)*P.at(0, comp, x);
@@ -715,6 +727,9 @@ BdryRegion bdry_region(const ibamr_plan* P, const BdryOp& op, const int* bx, boo
         R.hi[d] = bx[5 + d] + more;
         n[d] = R.hi[d] - R.lo[d] + 1;
     }
+    auto layers = [&](int d, int up) -> long {
+        return bd_inward(up, up ? Q.ihi[d] : Q.ilo[d], bx[2 + d], bx[5 + d]);
+    };
     // along a normal axis d of an edge or corner: the box, and its mirror image inside
     // (cell data) or the two values that extrapolate (side data)
     auto inward = [&](int d, int up) {
@@ -764,7 +779,7 @@ BdryRegion bdry_region(const ibamr_plan* P, const BdryOp& op, const int* bx, boo
         int e, n1, n2, u1, u2;
         bd_edge(loc, &e, &n1, &n2, &u1, &u2);
         if (op.kind == B_CC_EDGE)
-            *count = n[e] * (n[n1] * n[n2] + (adjoint ? n[n1] + n[n2] : 0));
+            *count = n[e] * (adjoint ? layers(n1, u1) * layers(n2, u2) + n[n1] + n[n2] : n[n1] * n[n2]);
         else
             *count = n[e] * n[op.comp] * (adjoint ? 1 : n[op.comp == n1 ? n2 : n1]);
         inward(n1, u1);
@@ -773,12 +788,14 @@ BdryRegion bdry_region(const ibamr_plan* P, const BdryOp& op, const int* bx, boo
     }
     case B_CC_CORNER:
     case B_SC_CORNER:
-        if (op.kind == B_CC_CORNER)
+        if (op.kind == B_CC_CORNER && adjoint)
         {
-            *count = n[0] * n[1] * n[2];
-            if (adjoint)
-                for (int d = 0; d < nd; ++d) *count += n[d];
+            *count = 1;
+            for (int d = 0; d < nd; ++d) *count *= layers(d, (loc >> d) & 1);
+            for (int d = 0; d < nd; ++d) *count += n[d];
         }
+        else if (op.kind == B_CC_CORNER)
+            *count = n[0] * n[1] * n[2];
         else
             *count = adjoint ? n[op.comp] : n[0] * n[1] * n[2];
         for (int d = 0; d < nd; ++d) inward(d, (loc >> d) & 1);
