@@ -817,23 +817,23 @@ std::vector<std::vector<BdryOp>> bdry_stages(const ibamr_plan* P, const std::vec
     const int phases_adj[4] = {3, 2, 10, 11}, phases_fwd[4] = {11, 10, 2, 3};
     struct Done
     {
-        int comp, stage;
+        int stage;
         BdryRegion r;
     };
     for (const int4& pl : patches)
     {
-        std::vector<Done> done;
+        std::vector<std::vector<Done>> done(side ? nd : P->depth);  // per component
         auto put = [&](int box, int kind, int comp) {
             BdryOp op{pl.x, box, kind, comp, 0};
             const BdryRegion r = bdry_region(P, op, &boxes[8 * (size_t)box], adjoint, &op.count);
             int st = 0;
-            for (const Done& o : done)
+            for (const Done& o : done[comp])
             {
-                bool meet = o.comp == comp;
+                bool meet = true;
                 for (int d = 0; d < nd; ++d) meet = meet && r.lo[d] <= o.r.hi[d] && o.r.lo[d] <= r.hi[d];
                 if (meet) st = std::max(st, o.stage + 1);
             }
-            done.push_back(Done{comp, st, r});
+            done[comp].push_back(Done{st, r});
             if ((int)stages.size() <= st) stages.resize(st + 1);
             if (op.count > 0) stages[st].push_back(op);
         };
@@ -1153,16 +1153,23 @@ static int set_physical_boundary(ibamr_plan* P, const ibamr_bdry_box* boxes, int
     P->bdry_box_d = reinterpret_cast<int*>(P->bdry_mem_d + at_box);
     P->bdry_coef_d = reinterpret_cast<double*>(P->bdry_mem_d + at_coef);
     P->bdry_coef_off_d = reinterpret_cast<long*>(P->bdry_mem_d + at_off);
-    HIP_OK(hipMemcpy(P->bdry_coef_d, cf.data(), sizeof(double) * cf.size(), hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(P->bdry_coef_off_d, cfo.data(), sizeof(long) * cfo.size(), hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(P->bdry_box_d, bx.data(), sizeof(int) * bx.size(), hipMemcpyHostToDevice));
+    // two copies (a caller whose coefficients change in time sets them every step):
+    // the coefficients, and the other tables behind them
+    std::vector<char> mem(bytes - at_off);
+    auto put = [&](size_t at, const auto& v) {
+        if (!v.empty()) std::memcpy(mem.data() + (at - at_off), v.data(), sizeof(v[0]) * v.size());
+    };
+    put(at_off, cfo);
+    put(at_box, bx);
     for (int m = 0; m < 2; ++m)
     {
         P->bdry_ops_d[m] = reinterpret_cast<BdryOp*>(P->bdry_mem_d + at_ops[m]);
         P->bdry_blocks_d[m] = reinterpret_cast<int2*>(P->bdry_mem_d + at_blocks[m]);
-        HIP_OK(hipMemcpy(P->bdry_ops_d[m], ops[m].data(), sizeof(BdryOp) * ops[m].size(), hipMemcpyHostToDevice));
-        HIP_OK(hipMemcpy(P->bdry_blocks_d[m], blocks[m].data(), sizeof(int2) * blocks[m].size(), hipMemcpyHostToDevice));
+        put(at_ops[m], ops[m]);
+        put(at_blocks[m], blocks[m]);
     }
+    HIP_OK(hipMemcpy(P->bdry_coef_d, cf.data(), sizeof(double) * cf.size(), hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(P->bdry_mem_d + at_off, mem.data(), mem.size(), hipMemcpyHostToDevice));
     P->nbdry_patches = (int)pl.size();
     return IBAMR_OK;
 }
