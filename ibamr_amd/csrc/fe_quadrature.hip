@@ -147,29 +147,26 @@ __global__ void k_fe_qp(int ndim, int nvars, int nelem, int nbasis, int nqp, int
 // FEDataManager::interpWeighted after the interpolation to the quadrature
 // points (FEDataManager.cpp:2009-2061, integrate_elem_rhs :1569-1606): every
 // element forms rhs[k][i] = sum_q U_qp[q][i] * (phi[k][q] * JxW[q]) (q in order
-// from 0.0) and adds it to its nodes in element order.  FE_NODE_LANES lanes per
-// node take its (element, basis) list, in element order, that many entries at a
-// time: each sums one entry's r, then all add the entries' sums in list order, so
-// each node value is that same sequence of operations.  Bound by the latency of
-// the loads of the quadrature points' values: one thread per node left 1.8
-// wavefronts per SIMD for 118 k nodes (hexahedra of 8 points, 3 variables:
-// 92 us; 113 us with one thread per node); now by the lines that a load of 64
-// entries' values touches.
-constexpr int FE_NODE_LANES = 8;
-template <typename TU>
+// from 0.0) and adds it to its nodes in element order.  LANES lanes per node take
+// its (element, basis) list, in element order, that many entries at a time: each
+// sums one entry's r, then all add the entries' sums in list order, so each node
+// value is that same sequence of operations.  Bound by the latency of the loads of
+// the quadrature points' values, or by instructions where lanes have no entry
+// (fe_node_lanes).
+template <typename TU, int LANES>
 __global__ void k_fe_node_rhs(int nvars, int nnodes, int nqp, const int* __restrict__ start,
                               const int2* __restrict__ ent, const double* __restrict__ phi,
                               const double* __restrict__ JxW, const TU* __restrict__ U_qp, double* __restrict__ F,
                               int overwrite)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)nnodes * FE_NODE_LANES) return;
-    const int v = (int)(t / FE_NODE_LANES), l = threadIdx.x % FE_NODE_LANES;
+    if (t >= (long)nnodes * LANES) return;
+    const int v = (int)(t / LANES), l = threadIdx.x % LANES;
     double acc[FE_MAX_VARS];
 #pragma unroll
     for (int i = 0; i < FE_MAX_VARS; ++i) acc[i] = overwrite ? 0.0 : (i < nvars ? F[(size_t)v * nvars + i] : 0.0);
     const int j1 = start[v + 1];
-    for (int j0 = start[v]; j0 < j1; j0 += FE_NODE_LANES)
+    for (int j0 = start[v]; j0 < j1; j0 += LANES)
     {
         double r[FE_MAX_VARS];
 #pragma unroll
@@ -186,11 +183,11 @@ __global__ void k_fe_node_rhs(int nvars, int nnodes, int nqp, const int* __restr
                     if (i < nvars) r[i] = r[i] + (double)u[i] * p;
             }
         }
-        const int m = min(FE_NODE_LANES, j1 - j0);
+        const int m = min(LANES, j1 - j0);
         for (int j = 0; j < m; ++j)
 #pragma unroll
             for (int i = 0; i < FE_MAX_VARS; ++i)
-                if (i < nvars) acc[i] = acc[i] + __shfl(r[i], j, FE_NODE_LANES);
+                if (i < nvars) acc[i] = acc[i] + __shfl(r[i], j, LANES);
     }
     if (l != 0) return;
 #pragma unroll
@@ -368,6 +365,22 @@ __global__ void k_fe_adaptive_orders(int type, int ndim, int nelem, int nbasis, 
 }
 } // namespace
 
+// Lanes per node of k_fe_node_rhs (the result does not depend on them).  8 where
+// their threads are no more than the GPU holds at once (256 CUs x 2048: only latency
+// counts), else by the quadrature points behind a node.  Time with 1 / 2 / 8 lanes,
+// us: one-point quadrilaterals (4 points per node, 491 k nodes, 1 variable) 8 / 10 /
+// 23, EDGE3 with 3 points (4.5; 2 M, 2) 42 / 41 / 140; one-point triangles (6; 491 k,
+// 3) 48 / 29 / 36, one-point hexahedra (8; 358 k, 3) 25 / 22 / 30, EDGE2 with 5 points
+// (10; 1 M, 2) 159 / 51 / 101, quadrilaterals with 4 points (16; 491 k, 2) 102 / 36 /
+// 58; triangles with 3 points (18; 491 k, 3) 389 / 208 / 69, hexahedra with 8 points
+// (64; 358 k, 3) 995 / 297 / 227.
+static int fe_node_lanes(long nnodes, long nentries, long nqp)
+{
+    if (nnodes * 8 <= 256L * 2048) return 8;
+    const long points = nentries * nqp;
+    return points < 5 * nnodes ? 1 : points < 17 * nnodes ? 2 : 8;
+}
+
 struct ibamr_fe_mesh
 {
     int nelem = 0, nbasis = 0, nnodes = 0;
@@ -435,14 +448,19 @@ int ibamr_fe_integrate_rhs(const ibamr_fe_mesh* m, int nvars, int nqp, const dou
     if (!F_nodes || (m->nelem > 0 && (!phi || !JxW || !U_qp))) return set_error(IBAMR_ERR_INVALID, "null argument");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int B = 256;
-    const dim3 G((unsigned)(((long)m->nnodes * FE_NODE_LANES + B - 1) / B));
     const int ow = mode == IBAMR_SPREAD_OVERWRITE ? 1 : 0;
+    const int lanes = fe_node_lanes(m->nnodes, (long)m->nelem * m->nbasis, nqp);
+    const dim3 G((unsigned)(((long)m->nnodes * lanes + B - 1) / B));
+    auto go = [&](auto tag) {
+        using TU = decltype(tag);
+        const auto kernel = lanes == 1 ? k_fe_node_rhs<TU, 1> : lanes == 2 ? k_fe_node_rhs<TU, 2> : k_fe_node_rhs<TU, 8>;
+        hipLaunchKernelGGL(kernel, G, dim3(B), 0, s, nvars, m->nnodes, nqp, m->start, m->ent, phi, JxW,
+                           static_cast<const TU*>(U_qp), F_nodes, ow);
+    };
     if (u_precision == IBAMR_FP64)
-        hipLaunchKernelGGL(k_fe_node_rhs<double>, G, dim3(B), 0, s, nvars, m->nnodes, nqp, m->start, m->ent, phi, JxW,
-                           static_cast<const double*>(U_qp), F_nodes, ow);
+        go((double)0);
     else
-        hipLaunchKernelGGL(k_fe_node_rhs<float>, G, dim3(B), 0, s, nvars, m->nnodes, nqp, m->start, m->ent, phi, JxW,
-                           static_cast<const float*>(U_qp), F_nodes, ow);
+        go((float)0);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(IBAMR_ERR_DEVICE, std::string("k_fe_node_rhs: ") + hipGetErrorString(e));
     return IBAMR_OK;
