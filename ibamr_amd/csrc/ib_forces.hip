@@ -29,6 +29,7 @@
 #include <cfloat>
 #include <map>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace ibamr
@@ -91,15 +92,22 @@ struct ForceArgs
     const double *t_K, *t_E, *t_X0;
 };
 
-// Bound by memory: per node of a ring with springs, beams and a target point at
-// every 4th node about 220 bytes of lists, parameters, positions and force.  1.5 M
-// nodes FP64: 85 us a call; 139 us as a spring, a beam and a gather kernel.
-template <int NDIM, typename TF, typename TU>
+// LANES lanes per node take its list that many entries at a time: each evaluates one
+// entry, then all add the entries' forces in list order.  Nodes of few entries are
+// bound by memory (per node of a ring with springs, beams and a target point at every
+// 4th node about 220 bytes of lists, parameters, positions and force; 1.5 M nodes FP64:
+// 85 us a call, 139 us as a spring, a beam and a gather kernel), nodes of many by the
+// latency of the chain start -> entry -> element -> position.  1 / 2 / 8 lanes, us:
+// springs of a ring (2 entries a node, 10^6 nodes) 19 / 18 / 51, beams (3) 30 / 30 / 63,
+// spring networks of valence 12 and 26 (200 k nodes) 115 / 90 / 47 and 306 / 220 / 107
+// (287 as a spring and a gather kernel).
+template <int NDIM, typename TF, typename TU, int LANES>
 __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* __restrict__ X,
                                                      const TU* __restrict__ U, TF* __restrict__ F, int overwrite)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= a.n) return;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long)a.n * LANES) return;
+    const int v = (int)(t / LANES), l = threadIdx.x % LANES;
     double acc[NDIM], Xv[NDIM];
 #pragma unroll
     for (int d = 0; d < NDIM; ++d)
@@ -107,9 +115,8 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
         acc[d] = 0.0;
         Xv[d] = X[(size_t)NDIM * v + d];
     }
-    const int e1 = a.start[v + 1];
-    for (int e = a.start[v]; e < e1; ++e)
-    {
+    // add(d, f_d) with what entry e adds to the node's force; false: nothing (skipped)
+    auto entry = [&](int e, auto add) {
         int role, k;
         if (a.packed)
         {
@@ -138,7 +145,7 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
             double R2 = D[0] * D[0] + D[1] * D[1];
             if (NDIM == 3) R2 = R2 + D[NDIM - 1] * D[NDIM - 1];
             const double R = sqrt(R2);
-            if (R < DBL_EPSILON) continue;
+            if (R < DBL_EPSILON) return false;
             double T;
             if (a.s_law)
             {
@@ -151,8 +158,8 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
 #pragma unroll
             for (int d = 0; d < NDIM; ++d)
             {
-                const double f = T_over_R * D[d];
-                acc[d] = master ? acc[d] + f : acc[d] - f;
+                const double q = T_over_R * D[d];
+                add(d, master ? q : -q);
             }
         }
         else if (role <= R_BEAM_PREV)
@@ -165,8 +172,8 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
 #pragma unroll
             for (int d = 0; d < NDIM; ++d)
             {
-                const double f = K * (((X[in + d] + X[ip + d]) - 2.0 * X[im + d]) - a.b_c[(size_t)NDIM * k + d]);
-                acc[d] = role == R_BEAM_MASTER ? acc[d] + 2.0 * f : acc[d] - f;
+                const double q = K * (((X[in + d] + X[ip + d]) - 2.0 * X[im + d]) - a.b_c[(size_t)NDIM * k + d]);
+                add(d, role == R_BEAM_MASTER ? 2.0 * q : -q);
             }
         }
         else  // target point (IBStandardForceGen.cpp:1285-1288)
@@ -176,9 +183,35 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
             for (int d = 0; d < NDIM; ++d)
             {
                 const double u = U ? (double)U[(size_t)NDIM * v + d] : 0.0;
-                acc[d] = acc[d] + (K * (a.t_X0[(size_t)NDIM * k + d] - Xv[d]) - E * u);
+                add(d, K * (a.t_X0[(size_t)NDIM * k + d] - Xv[d]) - E * u);
             }
         }
+        return true;
+    };
+    const int e1 = a.start[v + 1];
+    if constexpr (LANES == 1)
+    {
+        for (int e = a.start[v]; e < e1; ++e) entry(e, [&](int d, double f) { acc[d] = acc[d] + f; });
+    }
+    else
+    {
+        for (int e0 = a.start[v]; e0 < e1; e0 += LANES)
+        {
+            double f[NDIM] = {};
+            const int some = e0 + l < e1 && entry(e0 + l, [&](int d, double g) { f[d] = g; }) ? 1 : 0;
+            const int m = min(LANES, e1 - e0);
+            for (int j = 0; j < m; ++j)
+            {
+                const int take = __shfl(some, j, LANES);
+#pragma unroll
+                for (int d = 0; d < NDIM; ++d)
+                {
+                    const double g = __shfl(f[d], j, LANES);
+                    acc[d] = take ? acc[d] + g : acc[d];
+                }
+            }
+        }
+        if (l != 0) return;
     }
     // F += F_ghost (VecAXPY with alpha 1, :300), or F = F_ghost
 #pragma unroll
@@ -220,6 +253,7 @@ struct ibamr_forces
     int* start = nullptr;
     int* ent = nullptr;
     bool packed = true;
+    int lanes = 1;  // lanes per node of k_node_forces
 };
 
 extern "C" {
@@ -299,6 +333,12 @@ int ibamr_forces_create(ibamr_forces** out, int ndim, int npoints, int nsprings,
 
     ibamr_forces* f = new ibamr_forces();
     f->packed = packed;
+    // 8 lanes per node for lists of 12 entries and more on average, or where one is so
+    // long that it takes longer than all others (one hub of 1000 springs: 535 us with one
+    // lane, 235 with 8; see k_node_forces)
+    size_t longest = 0;
+    for (const auto& l : lists) longest = std::max(longest, l.size());
+    f->lanes = nent >= 12 * (size_t)npoints || longest >= 256 ? 8 : 1;
     f->ndim = ndim;
     f->n = npoints;
     f->ns = nsprings;
@@ -406,37 +446,28 @@ int ibamr_forces_compute(ibamr_forces* f, void* F, int f_precision, const double
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int B = 256;
     const int ow = mode == IBAMR_SPREAD_OVERWRITE ? 1 : 0;
-    const dim3 grid((f->n + B - 1) / B);
-    const bool u32 = U && u_precision == IBAMR_FP32C;
+    const int lanes = f->lanes;
+    const dim3 grid((unsigned)(((long)f->n * lanes + B - 1) / B));
     const ForceArgs a{f->n,   f->start, f->ent, f->packed ? 1 : 0, f->s_m, f->s_s, f->s_law, f->s_off, f->s_par, f->b_m,
                       f->b_n, f->b_p,   f->b_K, f->b_c,            f->t_K, f->t_E, f->t_X0};
-#define FORCES(NDIM, TF, TU)                                                                                 \
-    hipLaunchKernelGGL((k_node_forces<NDIM, TF, TU>), grid, dim3(B), 0, s, a, X, static_cast<const TU*>(U),  \
-                       static_cast<TF*>(F), ow)
-#define FORCES_BY_DIM(TF, TU)          \
-    do                                 \
-    {                                  \
-        if (f->ndim == 3)              \
-            FORCES(3, TF, TU);         \
-        else                           \
-            FORCES(2, TF, TU);         \
-    } while (0)
-    if (f_precision == IBAMR_FP64)
-    {
-        if (u32)
-            FORCES_BY_DIM(double, float);
+    auto go = [&](auto dim, auto tf, auto tu) {
+        using TF = decltype(tf);
+        using TU = decltype(tu);
+        constexpr int NDIM = decltype(dim)::value;
+        const auto kernel = lanes == 8 ? k_node_forces<NDIM, TF, TU, 8> : k_node_forces<NDIM, TF, TU, 1>;
+        hipLaunchKernelGGL(kernel, grid, dim3(B), 0, s, a, X, static_cast<const TU*>(U), static_cast<TF*>(F), ow);
+    };
+    auto by_type = [&](auto dim) {
+        const bool u32 = U && u_precision == IBAMR_FP32C;
+        if (f_precision == IBAMR_FP64)
+            u32 ? go(dim, 0.0, 0.0f) : go(dim, 0.0, 0.0);
         else
-            FORCES_BY_DIM(double, double);
-    }
+            u32 ? go(dim, 0.0f, 0.0f) : go(dim, 0.0f, 0.0);
+    };
+    if (f->ndim == 3)
+        by_type(std::integral_constant<int, 3>());
     else
-    {
-        if (u32)
-            FORCES_BY_DIM(float, float);
-        else
-            FORCES_BY_DIM(float, double);
-    }
-#undef FORCES_BY_DIM
-#undef FORCES
+        by_type(std::integral_constant<int, 2>());
     F_HIP(hipGetLastError());
     return IBAMR_OK;
 }
