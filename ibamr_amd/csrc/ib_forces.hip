@@ -222,6 +222,12 @@ __global__ __launch_bounds__(256) void k_node_forces(ForceArgs a, const double* 
     }
 }
 
+__global__ void k_copy_positions(long n, const double* __restrict__ X, double* __restrict__ out)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = X[i];
+}
+
 template <typename T>
 int dev_copy(T** dst, const T* src, size_t n)
 {
@@ -252,6 +258,7 @@ struct ibamr_forces
     double *t_K = nullptr, *t_E = nullptr, *t_X0 = nullptr;
     int* start = nullptr;
     int* ent = nullptr;
+    double* Xc = nullptr;  // [n][ndim] positions while F is written over them
     bool packed = true;
     int lanes = 1;  // lanes per node of k_node_forces
 };
@@ -263,7 +270,7 @@ int ibamr_forces_destroy(ibamr_forces* f)
     if (!f) return IBAMR_OK;
     for (void* p : {(void*)f->s_m, (void*)f->s_s, (void*)f->s_law, (void*)f->s_off, (void*)f->s_par, (void*)f->b_m, (void*)f->b_n,
                     (void*)f->b_p, (void*)f->b_K, (void*)f->b_c, (void*)f->t_i, (void*)f->t_K, (void*)f->t_E,
-                    (void*)f->t_X0, (void*)f->start, (void*)f->ent})
+                    (void*)f->t_X0, (void*)f->start, (void*)f->ent, (void*)f->Xc})
         dfree(p);
     delete f;
     return IBAMR_OK;
@@ -371,6 +378,10 @@ int ibamr_forces_create(ibamr_forces** out, int ndim, int npoints, int nsprings,
     chk(dev_copy(&f->t_X0, target_X0, (size_t)ntargets * ndim));
     chk(dev_copy(&f->start, start.data(), start.size()));
     chk(dev_copy(&f->ent, ent.data(), ent.size()));
+    // here and not at its first use, which may be under capture
+    if (rc == IBAMR_OK && nsprings + nbeams > 0 &&
+        hipMalloc(&f->Xc, sizeof(double) * (size_t)npoints * ndim) != hipSuccess)
+        rc = set_error(IBAMR_ERR_DEVICE, "hipMalloc of position scratch failed");
     if (rc != IBAMR_OK)
     {
         ibamr_forces_destroy(f);
@@ -446,6 +457,16 @@ int ibamr_forces_compute(ibamr_forces* f, void* F, int f_precision, const double
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int B = 256;
     const int ow = mode == IBAMR_SPREAD_OVERWRITE ? 1 : 0;
+    // springs and beams read other nodes' positions: from a copy where F lies over X
+    const size_t nv = (size_t)f->n * f->ndim;
+    const char *f0 = static_cast<const char*>(F), *f1 = f0 + nv * (f_precision == IBAMR_FP64 ? 8 : 4);
+    const char *x0 = reinterpret_cast<const char*>(X), *x1 = x0 + nv * 8;
+    if (f->Xc && f0 < x1 && x0 < f1)
+    {
+        hipLaunchKernelGGL(k_copy_positions, dim3((unsigned)((nv + B - 1) / B)), dim3(B), 0, s, (long)nv, X, f->Xc);
+        F_HIP(hipGetLastError());
+        X = f->Xc;
+    }
     const int lanes = f->lanes;
     const dim3 grid((unsigned)(((long)f->n * lanes + B - 1) / B));
     const ForceArgs a{f->n,   f->start, f->ent, f->packed ? 1 : 0, f->s_m, f->s_s, f->s_law, f->s_off, f->s_par, f->b_m,

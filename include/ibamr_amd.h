@@ -421,8 +421,8 @@ int ibamr_forces_create(ibamr_forces** forces, int ndim, int npoints, int nsprin
  * IBAMR_SPREAD_ACCUMULATE) or = (IBAMR_SPREAD_OVERWRITE) the force at positions X
  * (device, double); U (device, [n][ndim], double for u_precision IBAMR_FP64 or
  * float for IBAMR_FP32C, read as double; may be NULL = at rest) feeds the target
- * point damping.  Forces are summed in double either way.  Kernels only
- * (graph-safe). */
+ * point damping.  Forces are summed in double either way.  F may lie over X: all
+ * forces are those of the positions before the call.  Kernels only (graph-safe). */
 int ibamr_forces_compute(ibamr_forces* forces, void* F, int f_precision, const double* X, const void* U,
                          int u_precision, int mode, void* stream);
 int ibamr_forces_destroy(ibamr_forces* forces);
