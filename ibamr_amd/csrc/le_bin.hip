@@ -20,6 +20,7 @@ struct BinArgs
     int bin;
     int nmem;
     int ksub;   // bits of the plane-in-bin part of a key (0: bins only)
+    int* nactive;  // cleared for k_bin_bounds (null: not counted)
     int* keys;
     int4* cell;  // getCellIndex of every point, in the caller's order
 };
@@ -30,6 +31,7 @@ template <int NDIM>
 __global__ void k_bin_keys(BinArgs a)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0 && a.nactive) *a.nactive = 0;
     if (p >= a.n) return;
     int c[3] = {0, 0, 0};
     int raw[3] = {0, 0, 0};
@@ -284,8 +286,11 @@ void radix_pass(const ibamr_plan* P, const int* kin, const int* vin, int n, int 
 
 // start[b] = first sorted position whose key is >= b, for b in [0, m] (keys in
 // [0, m)): one binary search per bin, so the work per thread stays bounded
-// however the points are spread over the bins.
-__global__ void k_bin_bounds(const int* __restrict__ keys_sorted, int n, int m, int ksub, int* __restrict__ start)
+// however the points are spread over the bins.  nactive (if not null) counts the
+// superbins (8 bins, before the sentinel m - 1) that hold points: one atomic per
+// wavefront that has any, into a counter that k_bin_keys cleared.
+__global__ void k_bin_bounds(const int* __restrict__ keys_sorted, int n, int m, int ksub, int* __restrict__ start,
+                             int* __restrict__ nactive)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b > m) return;
@@ -299,6 +304,11 @@ __global__ void k_bin_bounds(const int* __restrict__ keys_sorted, int n, int m, 
             hi = mid;
     }
     start[b] = lo;
+    if (!nactive) return;
+    // the first point at or after the superbin's first bin lies in one of its bins
+    const bool some = (b & 7) == 0 && b < m - 1 && lo < n && (keys_sorted[lo] >> ksub) < b + 8;
+    const unsigned long long w = __ballot(some);
+    if (w && (threadIdx.x & 63) == __builtin_ctzll(w)) atomicAdd(nactive, __popcll(w));
 }
 
 // out[ndim * p + d] = coordinate d of point p's cell (caller's order)
@@ -400,6 +410,7 @@ int ibamr_plan_bin_async(ibamr_plan* P, const double* X, int npoints, void* stre
     a.bin = P->bin;
     a.nmem = P->nmem;
     a.ksub = P->ksub;
+    a.nactive = P->nactive_d;
     a.keys = P->keys_d;
     a.cell = P->cell_d;
     const int G = (npoints + B - 1) / B;
@@ -415,7 +426,7 @@ int ibamr_plan_bin_async(ibamr_plan* P, const double* X, int npoints, void* stre
         if (rc != IBAMR_OK) return rc;
     }
     hipLaunchKernelGGL(k_bin_bounds, dim3((m + 1 + B - 1) / B), dim3(B), 0, s, P->keys_sorted_d, npoints, m,
-                       P->ksub, P->bin_start_d);
+                       P->ksub, P->bin_start_d, P->nactive_d);
     HIP_OK(hipGetLastError());
     // idx_d is free once the sort is done: it now holds the inverse permutation
     hipLaunchKernelGGL(k_gather_cells, dim3(G), dim3(B), 0, s, P->perm_d, P->cell_d, npoints, P->cell_sorted_d,

@@ -40,6 +40,7 @@ struct InterpArgs
     int lev_lo[3];
     // 3-D: superbins with a static owner and block (see build_superbin_owners)
     const int* sb_owner;
+    const int* nactive;  // superbins that hold points (I3_BY_POINTS)
     int sb_off[2][2];
     int sbc;         // cells per superbin edge
     int nsy;         // superbins along y
@@ -183,6 +184,22 @@ __global__ __launch_bounds__(256) void k_interp(InterpArgs<T> a)
 
 #include "le_interp3d.h"
 
+// f(cut) with the cut as a constant, over the cuts that interp3_cut gives this kernel
+// and precision.
+template <int KER, typename T, typename F>
+int with_cut(int cut, F f)
+{
+    using Whole = std::integral_constant<int, I3_WHOLE>;
+    using Halves = std::integral_constant<int, I3_HALVES>;
+    using ByPoints = std::integral_constant<int, I3_BY_POINTS>;
+    if constexpr (sizeof(T) == 4 || KER == K_PWL)
+        return f(Whole());
+    else if constexpr (KER == K_IB6)
+        return f(Halves());
+    else
+        return cut == I3_WHOLE ? f(Whole()) : cut == I3_HALVES ? f(Halves()) : f(ByPoints());
+}
+
 // Raises the dynamic LDS limit of the 3-D interpolation kernels of a plan's
 // kernel and precision (done once at plan creation, not per launch: the
 // launches may be captured into a HIP graph).
@@ -192,13 +209,22 @@ int interp_prepare(int ndim, int kernel, int precision)
     return dispatch(3, kernel, precision, [&](auto, auto ker, auto prec) -> int {
         using T = decltype(prec);
         constexpr int KER = decltype(ker)::value;
-        // the variant reading the set-up pass's stencils exists for FP32C only
-        const void* fs[2] = {reinterpret_cast<const void*>(&k_interp3<KER, T, false>), nullptr};
-        if constexpr (sizeof(T) == 4) fs[1] = reinterpret_cast<const void*>(&k_interp3<KER, T, true>);
-        for (const void* f : fs)
-            if (f)
-                HIP_OK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           interp3_lds_elems<KER, T>() * (int)sizeof(T)));
+        auto raise = [&](auto cut) -> int {
+            // the variant reading the set-up pass's stencils exists for FP32C only
+            constexpr int CUT = decltype(cut)::value;
+            const void* fs[2] = {reinterpret_cast<const void*>(&k_interp3<KER, T, false, CUT>), nullptr};
+            if constexpr (sizeof(T) == 4) fs[1] = reinterpret_cast<const void*>(&k_interp3<KER, T, true, CUT>);
+            for (const void* f : fs)
+                if (f)
+                    HIP_OK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               interp3_lds_elems<KER>(0) * (int)sizeof(T)));
+            return IBAMR_OK;
+        };
+        for (int cut : {I3_WHOLE, I3_HALVES, I3_BY_POINTS})
+        {
+            const int rc = with_cut<KER, T>(cut, raise);
+            if (rc != IBAMR_OK) return rc;
+        }
         return IBAMR_OK;
     });
 }
@@ -335,6 +361,7 @@ int ibamr_plan_interp(ibamr_plan* P, int slot, void* U, const double* X, void* s
             a.gcw[d] = P->data_gcw[d];
         }
         a.sb_owner = P->sb_owner_d;
+        a.nactive = P->nactive_d;
         for (int v = 0; v < 2; ++v)
             for (int i = 0; i < 2; ++i) a.sb_off[v][i] = P->sb_off[v][i];
         a.sbc = 2 * P->bin;
@@ -352,27 +379,23 @@ int ibamr_plan_interp(ibamr_plan* P, int slot, void* U, const double* X, void* s
         {
             // one workgroup per superbin (or half of one); LDS holds one staged block of the array
             // (the kernel's dynamic LDS limit is raised once, at plan creation)
-            const int elems = interp3_lds_elems<KER, T>();
+            const int nsb = P->nsb[0] * P->nsb[1] * P->nsb[2];
+            const int nrow = P->nsb[1] * P->nsb[2];
+            const int cut = interp3_cut(P->kernel, P->precision, nsb);
+            const int elems = interp3_lds_elems<KER>(cut == I3_HALVES ? 1 : 0);
             const int bytes = elems * (int)sizeof(T);
             const int trc = time_begin(P, 1, s, &t_end);
             if (trc != IBAMR_OK) return trc;
-            const int nsb = P->nsb[0] * P->nsb[1] * P->nsb[2];
-            const int nrow = P->nsb[1] * P->nsb[2];
-            constexpr int zs = interp3_zs<KER, T>();
-            const int per = ((nrow + 7) / 8 * P->nsb[0]) << zs;  // workgroups per XCD (see k_interp3)
-            if constexpr (sizeof(T) == 4)
-            {
-                if (a.st)  // the spread set-up's stencils of these positions
-                {
-                    hipLaunchKernelGGL((k_interp3<KER, T, true>), dim3(8 * per), dim3(I3_THREADS), bytes, s, a,
-                                       elems, nsb, P->nsb[0], zs);
-                    HIP_OK(hipGetLastError());
-                    if (t_end) HIP_OK(hipEventRecord(t_end, s));
-                    return IBAMR_OK;
-                }
-            }
-            hipLaunchKernelGGL((k_interp3<KER, T, false>), dim3(8 * per), dim3(I3_THREADS), bytes, s, a, elems, nsb,
-                               P->nsb[0], zs);
+            const int per = ((nrow + 7) / 8 * P->nsb[0]) << (cut == I3_WHOLE ? 0 : 1);  // workgroups per XCD (see k_interp3)
+            const int rc = with_cut<KER, T>(cut, [&](auto c) -> int {
+                constexpr int CUT = decltype(c)::value;
+                auto kernel = k_interp3<KER, T, false, CUT>;
+                if constexpr (sizeof(T) == 4)
+                    if (a.st) kernel = k_interp3<KER, T, true, CUT>;  // the spread set-up's stencils of these positions
+                hipLaunchKernelGGL(kernel, dim3(8 * per), dim3(I3_THREADS), bytes, s, a, elems, nsb, P->nsb[0]);
+                return IBAMR_OK;
+            });
+            if (rc != IBAMR_OK) return rc;
         }
         else
         {

@@ -2,8 +2,8 @@
 // le_interp.hip, which defines InterpArgs and Sum).
 //
 // Interpolation (k_interp3): one IBAMR_I3_THREADS-thread (512) workgroup per
-// superbin (2x2x2 bins = 16^3 cells) or half of one (interp3_zs).  For each array it finds the exact stencil extent of its
-// points, stages that block of the ghosted array into LDS with coalesced
+// superbin (2x2x2 bins = 16^3 cells) or half of one (interp3_cut).  For each array it
+// finds the exact stencil extent of its points, stages that block of the ghosted array into LDS with coalesced
 // loads, then each thread sums the W^3 stencil of its points from LDS.
 #pragma once
 
@@ -24,26 +24,39 @@ constexpr int interp3_edge()
     return 16 + KernelTraits<KER>::W;
 }
 
-// 1: a workgroup takes the lower or the upper half of a superbin (16 x 16 x 8 cells).
-// While a workgroup waits for its block or sums from it, another one on the CU can do
-// the other, if the LDS holds both: with 22^3 doubles (IB_6) it does not, with halves
-// it does, for 1.27 times the halo.  Halves against whole superbins: IB_6 FP64, 8.4 M
-// points on 512^3: 4325 / 4672 us; IB_4 FP64, 1 M points on 256^3: 160 / 168 us, 0.5 M
-// on 200^3: 83 / 93 us.  Not where the halo is all that changes: FP32C (three or four
-// blocks fit as they are) IB_6 512^3 1832 / 1394 us, IB_4 and BSPLINE_3 of a 384^3
-// level 231 / 217 and 169 / 164 us (but 42 / 58 us for BSPLINE_3, 0.5 M on 200^3);
-// PIECEWISE_LINEAR FP64, 300^3: 411 / 311 us (little to sum per staged value).
-template <int KER, typename T>
-constexpr int interp3_zs()
+// A workgroup takes a whole superbin, or its lower or upper half (16 x 16 x 8 cells).
+// Halves stage 1.2 times the values and pay a workgroup's latencies twice; they gain
+// where
+//   the LDS holds one whole block but two half blocks (22^3 doubles, IB_6), so that one
+//     workgroup sums while another waits for its block (us, halves / whole, FP64: 512^3,
+//     10^6 points on a shell 425 / 541, 4.2 M uniform 3617 / 3703; 256^3 shell 319 / 398;
+//     the most it loses is a shell on 160^3, 420 / 392).  Not BSPLINE_6, whose weights
+//     take the time (200^3, 2 M uniform: 923 / 729);
+//   few superbins hold points, so that whole ones leave CUs idle or one of them is the
+//     last to end: up to 128 (256 CUs), or up to 768 of 1280 points and more on average
+//     (IB_4 40^3, 3000 points 17 / 21; 10^6 points on a shell 160^3 184 / 269, 256^3 140 /
+//     149; 512 k points in a ball 160^3 80 / 137), but for BSPLINE_6 between 128 and 256
+//     (one whole block a CU; 10^6 points on a shell 160^3 609 / 542).
+// Elsewhere whole superbins: IB_4, 0.03 points a cell uniform 128^3 37 / 25, 512^3 2258 /
+// 1457; 0.25 a cell 128^3 64 / 52, 200^3 254 / 210.  FP32C (three or four blocks fit as
+// they are) IB_6 512^3 1832 / 1394, IB_4 and BSPLINE_3 of a 384^3 level 231 / 217 and
+// 169 / 164; PIECEWISE_LINEAR FP64, 300^3: 411 / 311 (little to sum per staged value).
+// How many superbins hold points is known on the device only (counted when the points
+// are binned): where it decides (I3_BY_POINTS) twice the workgroups are launched and
+// the second half ends at once if superbins are taken whole.  Up to 4096 superbins
+// (256^3) that costs 1 % at most, at 512^3 (20000 points on a shell) 33 of 123 us; there
+// superbins are whole (10^6 points 244 / 202).
+template <int KER>
+__device__ __forceinline__ bool interp3_halves(int nactive, int npoints)
 {
-    return KER != K_PWL && sizeof(T) == 8 ? 1 : 0;
+    return nactive <= 128 || (nactive > (KER == K_BS6 ? 256 : 128) && nactive <= 768 && npoints >= 1280 * nactive);
 }
 
 // A cut superbin's block has 8 cells less along z.
-template <int KER, typename T>
-constexpr int interp3_lds_elems()
+template <int KER>
+constexpr int interp3_lds_elems(int zs)
 {
-    return interp3_edge<KER>() * interp3_edge<KER>() * (interp3_edge<KER>() - 8 * interp3_zs<KER, T>());
+    return interp3_edge<KER>() * interp3_edge<KER>() * (interp3_edge<KER>() - 8 * zs);
 }
 
 // Owning patch of a sorted point: the patch whose selection box holds its
@@ -70,8 +83,8 @@ __device__ __forceinline__ int interp_owner(const InterpArgs<T>& a, int k, const
     return -1;
 }
 
-template <int KER, typename T, bool LD>
-__global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds_elems, int nsb, int nsx, int zs)
+template <int KER, typename T, bool LD, int CUT>
+__global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds_elems, int nsb, int nsx)
 {
     using KT = KernelTraits<KER>;
     constexpr int W = KT::W;
@@ -94,6 +107,7 @@ __global__ __launch_bounds__(I3_THREADS) void k_interp3(InterpArgs<T> a, int lds
     // rows in order: a row's superbins share their x halo in one L2, and every
     // XCD gets a share of every region of the point cloud.
     const int xi = (int)(blockIdx.x % 8), qi = (int)(blockIdx.x / 8);
+    const int zs = CUT == I3_BY_POINTS ? (interp3_halves<KER>(*a.nactive, a.n) ? 1 : 0) : CUT;  // 1: halves
     const int nqx = nsx << zs, qx = qi % nqx;
     const int sb = (xi + 8 * (qi / nqx)) * nsx + (qx >> zs);
     if (sb >= nsb) return;

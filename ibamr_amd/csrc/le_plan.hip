@@ -202,6 +202,7 @@ int ibamr_plan_destroy(ibamr_plan* P)
     dfree(P->rs_hist_d);
     dfree(P->rs_off_d);
     dfree(P->rs_total_d);
+    dfree(P->nactive_d);
     delete P;
     return IBAMR_OK;
 }
@@ -423,6 +424,8 @@ static int plan_create_impl(ibamr_plan** out, const ibamr_level_geom* L, const i
         PLAN_HIP(hipMalloc(&P->rs_hist_d, sizeof(int) * nrs));
         PLAN_HIP(hipMalloc(&P->rs_off_d, sizeof(int) * nrs));
         PLAN_HIP(hipMalloc(&P->rs_total_d, sizeof(int) << RS_MAX_BITS));
+        if (ndim == 3 && interp3_cut(k, C->precision, P->nsb[0] * P->nsb[1] * P->nsb[2]) == I3_BY_POINTS)
+            PLAN_HIP(hipMalloc(&P->nactive_d, sizeof(int)));
     }
 #undef PLAN_HIP
     if (ndim == 3)

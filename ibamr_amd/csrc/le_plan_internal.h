@@ -83,6 +83,21 @@ constexpr int RS_TILE = RS_THREADS * RS_ROUNDS;
 static_assert(RS_TILE <= 65535, "ranks inside a tile are 16-bit");
 
 
+// Superbins of the 3-D interpolation: whole, in halves, or as the binned points say
+// (le_interp3d.h)
+enum InterpCut : int
+{
+    I3_WHOLE = 0,
+    I3_HALVES = 1,
+    I3_BY_POINTS = 2
+};
+inline int interp3_cut(int kernel, int precision, int nsb)
+{
+    if (precision != IBAMR_FP64 || kernel == K_PWL) return I3_WHOLE;
+    if (kernel == K_IB6 || nsb <= 128) return I3_HALVES;
+    return nsb <= 4096 ? I3_BY_POINTS : I3_WHOLE;
+}
+
 // IndexUtilities::getCellIndex (IndexUtilities-inl.h:52-72; the level form
 // :226-243 passes the level's domain box and x range) along one axis, as a
 // double: the lower side's formula when X is at least as close to x_lower as to
@@ -188,6 +203,7 @@ struct ibamr_plan
     int* rs_hist_d = nullptr;          // [digits * blocks] (digit, block) counts
     int* rs_off_d = nullptr;           // [digits * blocks] each digit's exclusive scan over the blocks
     int* rs_total_d = nullptr;         // [digits] keys of each digit
+    int* nactive_d = nullptr;          // superbins that hold points, where I3_BY_POINTS; else null
     int ncells = 0;                    // cells of all patches (pcell_off_d's last entry)
     int* perm_d = nullptr;
     int4* cell_d = nullptr;
