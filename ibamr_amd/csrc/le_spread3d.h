@@ -818,10 +818,18 @@ __global__ __launch_bounds__(64, ZC <= 16 ? 4 : 3) void k_spread3b(SpreadArgs<do
                     }
                     static_for<0, W>([&](auto ic) IBAMR_INLINE { c[decltype(ic)::value] = c[decltype(ic)::value] * Fj; });
                     __builtin_amdgcn_sched_barrier(0);
+                    if (!KT::IB)  // over vol; one choice for the W quotients, which then run side by side
+                    {
+                        if (a.vol_div == 1)  // a power of two: the product rounds as the quotient does
+                            static_for<0, W>([&](auto ic) IBAMR_INLINE { c[decltype(ic)::value] = c[decltype(ic)::value] * rvol; });
+                        else if (newton)
+                            static_for<0, W>([&](auto ic) IBAMR_INLINE { c[decltype(ic)::value] = div_by(c[decltype(ic)::value], vol, rvol); });
+                        else
+                            static_for<0, W>([&](auto ic) IBAMR_INLINE { c[decltype(ic)::value] = c[decltype(ic)::value] / vol; });
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     static_for<0, W>([&](auto ic) IBAMR_INLINE {
                         constexpr int i = decltype(ic)::value;
-                        if (!KT::IB)  // over vol (a power of two: the product rounds as the quotient does)
-                            c[i] = a.vol_div == 1 ? c[i] * rvol : (newton ? div_by(c[i], vol, rvol) : c[i] / vol);
                         if constexpr (zz + i >= 0 && zz + i < ZC) acc[zz + i] = acc[zz + i] + c[i];
                     });
                 }
