@@ -160,7 +160,6 @@ namespace
 template <typename T>
 void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double* X, int mode, SpreadArgs<T>& a)
 {
-    a.tiles = P->tlists[P->tcur].d;
     a.patches = P->patches_d;
     a.arrays = reinterpret_cast<T* const*>(P->arrays_d[slot]);
     a.X = X;
@@ -241,7 +240,9 @@ bool shape_admissible(const ibamr_plan* P, const Shape& sh)
     return !sweep || n[0] * n[1] <= 64;
 }
 
-// Tiles of the given extents over every array of every patch (one depth component).
+// Tiles of the given extents over every array of every patch, of one depth component:
+// spread_cut asks how many tiles share the points' work, and every component has the
+// same points.
 long count_tiles(const ibamr_plan* P, const Shape& ext)
 {
     long total = 0;
@@ -266,15 +267,21 @@ long count_tiles(const ibamr_plan* P, const Shape& ext)
 // IB_4, 10^6 points on a shell: 1.18 against 1.79 ms; AMR level of 384^3 0.79
 // against 1.08 ms).  Fewer tiles than the GPU holds wavefronts (256 CUs x 16):
 // 8 values (40^3, 432 tiles: 29 against 40 us; 64^3 IB_6, 1568 tiles: 259 against
-// 357 us; at 8736 tiles 207 against 185 us).  More than 128 per SIMD: 24, which
-// visit a point in fewer tiles (512^3 IB_6: 9.4 against 10.5 ms; at 86 k tiles
-// 1.35 against 1.11 ms).
+// 357 us; at 8736 tiles 207 against 185 us; cell data of 8 components on 128^3, 2601
+// tiles each, 200 k points on a shell 709 against 831 us, 20 k uniform 129 against 94).
+// More than 128 tiles per SIMD: 24 for IB_4, IB_6 and BSPLINE_6, which then visit a
+// point in fewer tiles (512^3 IB_6: 9.4 against 10.5 ms, IB_4 5.1 against 5.8,
+// BSPLINE_6, 4.2 M points 7.9 against 9.0; at 86 k tiles IB_6 1.35 against 1.11 ms).
+// The others keep 16 (512^3, 8.4 M points BSPLINE_3 5.8 against 6.6 ms; 4.2 M
+// BSPLINE_4 4.6 against 5.1, BSPLINE_5 6.0 against 6.3; 2.1 M PIECEWISE_LINEAR 2.0
+// against 2.2): more of their time goes into the tiles' own values.
 int spread_cut(const ibamr_plan* P, const Shape& sh)
 {
     if (P->ndim != 3 || P->precision != IBAMR_FP64) return sh[2];
     if (sh[0] != 8 || sh[2] != 32) return 16;
     if (count_tiles(P, {8, 8, 16}) < 4096) return 8;
-    return count_tiles(P, {8, 8, 24}) >= (1L << 17) ? 24 : 16;
+    const bool tall = P->kernel == K_IB4 || P->kernel == K_IB6 || P->kernel == K_BS6;
+    return tall && count_tiles(P, {8, 8, 24}) >= (1L << 17) ? 24 : 16;
 }
 
 // Work list of one tile shape: every tile of every array of every patch.
@@ -327,6 +334,22 @@ int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
     return IBAMR_OK;
 }
 
+// Index of the work list a spread takes: the one chosen, but for an overwriting IB_4
+// spread of fewer than two points per tile of 24 values the list of 16 values: most
+// tiles then write zeros, and those of IB_4 run four to a SIMD, whose unfinished lines
+// of 24 planes no longer fit the L2 (512^3, 20000 points: 1.33 ms, 0.93 with 16 values;
+// 10^6 points 1.36 and 1.35; accumulating 0.31 and 0.37).
+int spread_list(const ibamr_plan* P, int mode)
+{
+    const TileList& tl = P->tlists[P->tcur];
+    if (P->kernel != K_IB4 || P->precision != IBAMR_FP64 || mode != IBAMR_SPREAD_OVERWRITE || tl.cut != 24 ||
+        P->npoints >= 2L * tl.n)
+        return P->tcur;
+    for (size_t i = 0; i < P->tlists.size(); ++i)
+        if (P->tlists[i].shape[0] == 8 && P->tlists[i].cut == 16) return (int)i;
+    return P->tcur;
+}
+
 int find_shape(const ibamr_plan* P, const int* shape)
 {
     for (size_t i = 0; i < P->tlists.size(); ++i)
@@ -376,6 +399,8 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
         constexpr int KER = decltype(ker)::value;
         SpreadArgs<T> a{};
         fill_spread_args<T>(P, slot, F, X, mode, a);
+        const TileList& tl = P->tlists[spread_list(P, mode)];
+        a.tiles = tl.d;
         if (P->npoints > 0)
         {
             const int B = 256;
@@ -419,7 +444,6 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
         hipEvent_t t_end;
         const int trc = time_begin(P, 0, s, &t_end);
         if (trc != IBAMR_OK) return trc;
-        const TileList& tl = P->tlists[P->tcur];
         if constexpr (NDIM == 3)
         {
             const dim3 G(tl.n), B(64);

@@ -1,0 +1,37 @@
+"""FP64 spread on a level of more than 2^17 tiles, where the work items' z extent
+depends on the kernel (24 values IB_4, IB_6 and BSPLINE_6, 16 the others), on the mode
+and on the number of points (IB_4, overwriting): bit for bit against the oracle on
+every list that a plan chooses between."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+import ibamr_amd as ia  # noqa: E402
+from test_gpu_parity import _dev, _oracle_spread  # noqa: E402
+from test_gpu_spread_batches import _points  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+N = 408
+
+
+@pytest.mark.parametrize("kernel,npts,modes", [("IB_4", 4000, (ia.OVERWRITE, ia.ACCUMULATE)),
+                                               ("IB_4", 300000, (ia.OVERWRITE,)), ("BSPLINE_6", 4000, (ia.OVERWRITE,)),
+                                               ("BSPLINE_3", 4000, (ia.OVERWRITE,))])
+def test_large_level(orc, kernel, npts, modes):
+    print("spread cut", kernel, npts, flush=True)
+    rng = np.random.default_rng(npts)
+    X = _points(rng, N, 500, npts)
+    F = rng.standard_normal(X.shape)
+    level = ia.Level.uniform_periodic(N, 3)
+    plan = ia.LevelPlan(level, kernel, ia.SIDE, ia.FP64, max_points=len(X))
+    shapes = [ia.array_shape(level, 0, plan.data_gcw, ia.SIDE, axis=a) for a in range(3)]
+    want = _oracle_spread(orc, level, plan, [np.zeros(s) for s in shapes], X, F, kernel)
+    plan.bin(_dev(X))
+    for mode in modes:
+        # accumulating into zeros: the same values as overwriting anything
+        f = [torch.full(s, 0.0 if mode == ia.ACCUMULATE else 3.0, dtype=torch.float64, device="cuda") for s in shapes]
+        plan.bind(0, f)
+        plan.spread(0, _dev(F), _dev(X), mode=mode)
+        for a, b in zip(f, want):
+            assert np.array_equal(a.cpu().numpy(), b), mode
+    plan.close()
