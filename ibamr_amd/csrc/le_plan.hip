@@ -178,7 +178,8 @@ int ibamr_plan_destroy(ibamr_plan* P)
     for (auto& v : P->tev)
         for (hipEvent_t e : v) (void)hipEventDestroy(e);
     dfree(P->patches_d);
-    for (TileList& t : P->tlists) dfree(t.d);
+    for (TileList& t : P->tlists)
+        if (t.same < 0) dfree(t.d);
     dfree(P->wt_d);
     dfree(P->sb_owner_d);
     dfree(P->st_d);

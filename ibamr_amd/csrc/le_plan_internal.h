@@ -64,6 +64,7 @@ struct TileList
     int n = 0;
     int shape[3] = {1, 1, 1};
     int cut = 1;  // z extent of the work items (a shape's tiles may be cut along z, see spread_cut)
+    int same = -1;  // index of the earlier list with the same work items, whose d this one uses; -1: its own
 };
 
 

@@ -293,10 +293,23 @@ int spread_cut(const ibamr_plan* P, const Shape& sh)
 // are rarely uniform, so contiguous eighths of the domain would leave some XCDs
 // idle), and all XCDs sweep the domain together, so the data they re-read is
 // recent in the shared last-level cache.
+// Shapes cut into the same work items (FP64 8 x 8 x 32 and 8 x 8 x 16 where 32 is cut to
+// 16) share one list.
 int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
 {
     std::vector<TileDesc> tiles;
     const Shape ext = P->ndim == 3 ? Shape{sh[0], sh[1], spread_cut(P, sh)} : Shape{S2_TILE, S2_TILE, 1};
+    for (size_t i = 0; &P->tlists[i] != &out; ++i)
+    {
+        const TileList& t = P->tlists[i];
+        if (t.same < 0 && t.shape[0] == sh[0] && t.shape[1] == sh[1] && t.cut == ext[2])
+        {
+            out = t;
+            out.same = (int)i;
+            for (int d = 0; d < 3; ++d) out.shape[d] = sh[d];
+            return IBAMR_OK;
+        }
+    }
     out.cut = ext[2];
     const int ncomp_tiles = P->centering == IBAMR_SIDE ? P->ndim : P->depth;
     std::vector<std::vector<TileDesc>> q(8);
@@ -563,6 +576,7 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
         {
             for (int d = 0; d < 3; ++d) shapes[3 * i + d] = P->tlists[i].shape[d];
             ms[i] = std::numeric_limits<float>::infinity();
+            if (P->tlists[i].same >= 0) continue;
             P->tcur = (int)i;
             const int r = ibamr_plan_spread(P, slot, F, X, IBAMR_SPREAD_OVERWRITE, stream);  // untimed
             if (r != IBAMR_OK) return r;
@@ -570,6 +584,7 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
         for (int round = 0; round < ROUNDS; ++round)
             for (size_t i = 0; i < ns; ++i)
             {
+                if (P->tlists[i].same >= 0) continue;
                 P->tcur = (int)i;
                 HIP_OK(hipEventRecord(e0, s));
                 for (int k = 0; k < reps; ++k)
@@ -583,6 +598,8 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
                 HIP_OK(hipEventElapsedTime(&t, e0, e1));
                 ms[i] = std::min(ms[i], t / reps);
             }
+        for (size_t i = 0; i < ns; ++i)  // a shared list has its owner's time
+            if (P->tlists[i].same >= 0) ms[i] = ms[P->tlists[i].same];
         for (size_t i = 0; i < ns; ++i)
             if (ms[i] < best_ms)
             {

@@ -473,14 +473,19 @@ int ibamr_plan_kernel_times(ibamr_plan* plan, double* spread_ms, int* nspread, d
 int ibamr_plan_info(const ibamr_plan* plan, int* ntiles, int* tile, int* nbins);
 
 /* Spread tile shape.  The spread's work is a list of tiles (boxes of grid
- * values of one array of one patch), one workgroup each; a plan builds the
- * work list of every shape built for its form when it is created and keeps
- * them until it is destroyed, so changing the shape only selects another list
- * (a HIP graph captured earlier keeps launching the shape it captured, which
- * stays valid).  Shapes (x, y, z extents; the first is the default):
- *   2-D: 16 x 16.
- *   3-D FP64: 8 x 8 grid lines times 32 or 16 z values held in registers, or
- *     16 x 4 grid lines times 32.
+ * values of one array of one patch), one wavefront for each tile or piece of
+ * it; a plan builds the work list of every shape built for its form when it is
+ * created and keeps them until it is destroyed, so changing the shape only
+ * selects another list (a HIP graph captured earlier keeps launching the shape
+ * it captured, which stays valid).  Shapes (x, y, z extents; the first is the
+ * default):
+ *   2-D: 16 x 16, in pieces of 8 x 8.
+ *   3-D FP64: 8 x 8 grid lines times 32 or 16 z values, or 16 x 4 grid lines
+ *     times 32.  The z values are held in registers, in pieces: 16 each, but 8
+ *     x 8 x 32 in pieces of 8 on levels of few tiles and of 24 on levels of very
+ *     many (there an overwriting spread may take pieces of 16).  Shapes whose
+ *     pieces are the same (8 x 8 x 32 in pieces of 16 and 8 x 8 x 16) share one
+ *     list.
  *   3-D FP32C: 8 x 8 grid lines times 16, 8 or 24 z values, or 16 x 4 times 16;
  *     and 8 x 8 grid lines times a z segment of 64, 128 or 256 values swept
  *     through a 16-value register window, layer of bins by layer (each point
@@ -495,7 +500,8 @@ int ibamr_plan_info(const ibamr_plan* plan, int* ntiles, int* tile, int* nbins);
  *   set_tile_shape / get_tile_shape: shape[3].
  *   set_tile_height / get_tile_height: the first shape with that z extent / the
  *     z extent of the shape in use.
- *   autotune: for each shape one untimed spread of F at X into the arrays
+ *   autotune: for each shape (shapes that share a list are timed once) one
+ *     untimed spread of F at X into the arrays
  *     bound to `slot` (IBAMR_SPREAD_OVERWRITE: their values are replaced), then
  *     3 rounds over all shapes of `reps` timed spreads each, and keeps the
  *     shape with the fastest round.  shapes[3*i .. 3*i+2] and ms[i] (capacity

@@ -35,3 +35,31 @@ def test_large_level(orc, kernel, npts, modes):
         for a, b in zip(f, want):
             assert np.array_equal(a.cpu().numpy(), b), mode
     plan.close()
+
+
+@pytest.mark.parametrize("n,shared", [(40, False), (104, True)])
+def test_shapes_with_the_same_pieces(orc, n, shared):
+    """8 x 8 x 32 in pieces of 16 and 8 x 8 x 16 are one list: timed once, each accepted
+    and reported under its name, the same bits."""
+    rng = np.random.default_rng(n)
+    X, kernel = _points(rng, n, 300, 2000), "IB_4"
+    F = rng.standard_normal(X.shape)
+    level = ia.Level.uniform_periodic(n, 3)
+    plan = ia.LevelPlan(level, kernel, ia.SIDE, ia.FP64, max_points=len(X))
+    f = [np.zeros(ia.array_shape(level, 0, plan.data_gcw, ia.SIDE, axis=a)) for a in range(3)]
+    want = _oracle_spread(orc, level, plan, f, X, F, kernel)
+    dev = [_dev(a) for a in f]
+    plan.bind(0, dev)
+    Xd, Fd = _dev(X), _dev(F)
+    plan.bin(Xd)
+    t = plan.autotune(0, Fd, Xd, reps=2)
+    assert sorted(t) == [(8, 8, 16), (8, 8, 32), (16, 4, 32)] and all(v > 0 for v in t.values())
+    assert (t[(8, 8, 32)] == t[(8, 8, 16)]) == shared
+    assert plan.tile_shape == min(t, key=t.get)
+    for sh in t:
+        plan.tile_shape = sh
+        assert plan.tile_shape == sh
+        plan.spread(0, Fd, Xd, mode=ia.OVERWRITE)
+        for a, b in zip(dev, want):
+            assert np.array_equal(a.cpu().numpy(), b), sh
+    plan.close()
