@@ -300,13 +300,12 @@ void radix_pass(const ibamr_plan* P, const int* kin, const int* vin, int n, int 
 // [0, m)): one binary search per bin, so the work per thread stays bounded
 // however the points are spread over the bins.  nactive (if not null) counts the
 // superbins (8 bins, before the sentinel m - 1) that hold points: one atomic per
-// wavefront that has any, into a counter that k_bin_keys cleared.
+// workgroup that has any, into a counter that k_bin_keys cleared.
 __global__ void k_bin_bounds(const int* __restrict__ keys_sorted, int n, int m, int ksub, int* __restrict__ start,
                              int* __restrict__ nactive)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b > m) return;
-    int lo = 0, hi = n;
+    int lo = 0, hi = b <= m ? n : 0;
     while (lo < hi)
     {
         const int mid = (lo + hi) >> 1;
@@ -315,12 +314,12 @@ __global__ void k_bin_bounds(const int* __restrict__ keys_sorted, int n, int m, 
         else
             hi = mid;
     }
-    start[b] = lo;
+    if (b <= m) start[b] = lo;
     if (!nactive) return;
     // the first point at or after the superbin's first bin lies in one of its bins
     const bool some = (b & 7) == 0 && b < m - 1 && lo < n && (keys_sorted[lo] >> ksub) < b + 8;
-    const unsigned long long w = __ballot(some);
-    if (w && (threadIdx.x & 63) == __builtin_ctzll(w)) atomicAdd(nactive, __popcll(w));
+    const int count = __syncthreads_count(some);
+    if (threadIdx.x == 0 && count > 0) atomicAdd(nactive, count);
 }
 
 // out[ndim * p + d] = coordinate d of point p's cell (caller's order)
