@@ -132,8 +132,8 @@ struct SpreadArgs
     int dom_lo[3], dom_hi[3];
     int pshift[3];
     double dx[3];
-    double rdx[3];  // FP64: 1 / dx
-    int dx_ok;      //       dx in div_by's range
+    double rdx[3];  // 1 / dx; NaN for a dx out of div_by's range, which takes every position as near a tile
+    int dx_ok;      // every dx in div_by's range
     double vol, rvol;
     int vol_div;   // FP64: 1: vol is a power of two, 2: quotients by vol from its reciprocal (div_by), 0: divisions
     int fdepth;
@@ -176,7 +176,11 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
         a.pshift[d] = P->pshift[d];
         a.dx[d] = P->dx[d];
         a.rdx[d] = 1.0 / P->dx[d];
-        if (P->dx[d] < 1e-60 || P->dx[d] > 1e60) a.dx_ok = 0;
+        if (P->dx[d] < 1e-60 || P->dx[d] > 1e60)
+        {
+            a.rdx[d] = std::numeric_limits<double>::quiet_NaN();
+            a.dx_ok = 0;
+        }
         a.gcw[d] = P->data_gcw[d];
     }
     a.bin = P->bin;

@@ -664,7 +664,7 @@ __global__ __launch_bounds__(64, ZC <= 16 ? 4 : 3) void k_spread3b(SpreadArgs<do
                     ok = ok && ci >= clo[d] && ci <= chi[d];
                     const float t =
                         (float)((nX[d] - xl[d]) * a.rdx[d] + (double)(o[d] * a.pshift[d] + P.ilo[d] - flo[d]));
-                    ok = ok && !(t < tlo) && !(t > thi[d]);
+                    ok = ok && !(t < tlo) && !(t > thi[d]);  // (true for NaN)
                 }
                 cq += 64;
                 if (cq < gtotal) fetch(cq);
