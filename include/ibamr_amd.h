@@ -351,8 +351,10 @@ int ibamr_fe_nodal_weight(int nnodes, int nvars, const void* V, int v_precision,
  * points that reach them; SAMRAI's accumulation leaves there only the patch's
  * own points' contributions, so on levels with several patches the two agree
  * where no other patch's points reach a patch's out-of-domain ghost cells.
- * set_physical_boundary validates the boxes (inside the ghost box) and copies
- * them to the device; the other two enqueue one kernel (graph-safe). */
+ * set_physical_boundary validates the boxes (inside the ghost box, edge and
+ * corner boxes anywhere outside the patch on their sides) and copies them to
+ * the device; the other two enqueue one kernel per stage of boxes that do not
+ * meet (graph-safe; six for side data of a 3-D patch with walls all around). */
 typedef struct
 {
     int patch;      /* patch index in the level */
