@@ -63,7 +63,7 @@ struct TileList
     TileDesc* d = nullptr;
     int n = 0;
     int shape[3] = {1, 1, 1};
-    int cut = 1;  // z extent of the work items (a shape's tiles may be cut along z, see spread_cut)
+    int cut = 1;  // extent of the work items: 3-D along z (spread_cut), 2-D their edge
     int same = -1;  // index of the earlier list with the same work items, whose d this one uses; -1: its own
 };
 
@@ -164,6 +164,7 @@ struct ibamr_plan
     PatchDev* patches_d = nullptr;
     std::vector<TileList> tlists;      // spread work lists, one per admissible tile shape (first: default)
     int tcur = 0;                      // the shape in use
+    TileList tsparse;                  // 2-D levels of many tiles: whole 16 x 16 tiles (spread_list); n = 0: none
     // FP32C 3-D: the stencils of the bin-ordered positions, set up once per
     // spread (k_point_weights): for axis d and variant v (v = 1: x_lower - dx/2,
     // the normal axis of side data) the first stencil index

@@ -203,7 +203,8 @@ void fill_spread_args(const ibamr_plan* P, int slot, const void* F, const double
 }
 
 // Spread tile shapes built for each form; the first is the default.
-//   2-D: 16 x 16, taken as four 8 x 8 work items (k_spread2).
+//   2-D: 16 x 16, taken as four 8 x 8 work items, or whole where few tiles have a point
+//     (k_spread2, spread_list).
 //   3-D: 8 x 8 or 16 x 4 grid lines (one per lane) times a column of z values
 //     in registers (k_spread3b FP64, k_spread3 FP32C); an FP64 tile is cut along z
 //     into work items (spread_cut).  FP32C keeps two register sets per z value (the
@@ -288,6 +289,10 @@ int spread_cut(const ibamr_plan* P, const Shape& sh)
     return tall && count_tiles(P, {8, 8, 24}) >= (1L << 17) ? 24 : 16;
 }
 
+// 2-D levels of at least this many 8 x 8 tiles also have a list of whole 16 x 16 tiles
+// (spread_list).
+constexpr long S2_MANY_TILES = 1L << 14;
+
 // Work list of one tile shape: every tile of every array of every patch.
 // XCD-aware launch order: workgroup i runs on XCD i % 8.  Tiles are grouped by
 // (patch, z row, y row), each group holding that row of every array, and the
@@ -299,14 +304,14 @@ int spread_cut(const ibamr_plan* P, const Shape& sh)
 // recent in the shared last-level cache.
 // Shapes cut into the same work items (FP64 8 x 8 x 32 and 8 x 8 x 16 where 32 is cut to
 // 16) share one list.
-int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
+int build_tiles(ibamr_plan* P, const Shape& sh, int cut, TileList& out)
 {
     std::vector<TileDesc> tiles;
-    const Shape ext = P->ndim == 3 ? Shape{sh[0], sh[1], spread_cut(P, sh)} : Shape{S2_TILE, S2_TILE, 1};
-    for (size_t i = 0; &P->tlists[i] != &out; ++i)
+    const Shape ext = P->ndim == 3 ? Shape{sh[0], sh[1], cut} : Shape{cut, cut, 1};
+    for (size_t i = 0; i < P->tlists.size() && &P->tlists[i] != &out; ++i)
     {
         const TileList& t = P->tlists[i];
-        if (t.same < 0 && t.shape[0] == sh[0] && t.shape[1] == sh[1] && t.cut == ext[2])
+        if (t.same < 0 && t.shape[0] == sh[0] && t.shape[1] == sh[1] && t.cut == cut)
         {
             out = t;
             out.same = (int)i;
@@ -314,7 +319,7 @@ int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
             return IBAMR_OK;
         }
     }
-    out.cut = ext[2];
+    out.cut = cut;
     const int ncomp_tiles = P->centering == IBAMR_SIDE ? P->ndim : P->depth;
     std::vector<std::vector<TileDesc>> q(8);
     size_t g = 0;
@@ -351,20 +356,35 @@ int build_tiles(ibamr_plan* P, const Shape& sh, TileList& out)
     return IBAMR_OK;
 }
 
-// Index of the work list a spread takes: the one chosen, but for an overwriting IB_4
-// spread of fewer than two points per tile of 24 values the list of 16 values: most
-// tiles then write zeros, and those of IB_4 run four to a SIMD, whose unfinished lines
-// of 24 planes no longer fit the L2 (512^3, 20000 points: 1.33 ms, 0.93 with 16 values;
-// 10^6 points 1.36 and 1.35; accumulating 0.31 and 0.37).
-int spread_list(const ibamr_plan* P, int mode)
+// The work list a spread takes: the one chosen, but for few points per tile
+//   IB_4 3-D, fewer than two per tile of 24 values, overwriting: the list of 16 values:
+//     most tiles then write zeros, and those of IB_4 run four to a SIMD, whose
+//     unfinished lines of 24 planes no longer fit the L2 (512^3, 20000 points: 1.33 ms,
+//     0.93 with 16 values; 10^6 points 1.36 and 1.35; accumulating 0.31 and 0.37).
+//   2-D, fewer than t^1.5 / 1024 at t tiles of 8 x 8 (1536 where an empty tile's values
+//     are not touched): whole 16 x 16 tiles, a quarter of the workgroups, since the
+//     launch and an empty tile's own steps are what it costs (FP64 IB_4, side: 2048^2,
+//     5000 points 45 against 95 us uniform, 34 against 77 on a circle; 4096^2, 20000 in
+//     a disc 126 against 321, 2 x 10^5 on a circle 224 against 312).  With more points
+//     the longest chain decides, and a 16 x 16 tile's is up to four times as long.
+//     Workgroups grow with t, the chain of points on a curve with their number over
+//     t^0.5, so the line is at t^1.5: 800^2, 3000 on a circle 17 against 19, 1400^2,
+//     10^4 34 and 41, 3 x 10^4 68 and 53; 2048^2, 6 x 10^4 99 and 91 (uniform 64 and
+//     141).  Accumulating 2048^2, 45000 on a circle 74 and 63, 5000 23 and 49.
+const TileList& spread_list(const ibamr_plan* P, int mode)
 {
     const TileList& tl = P->tlists[P->tcur];
-    if (P->kernel != K_IB4 || P->precision != IBAMR_FP64 || mode != IBAMR_SPREAD_OVERWRITE || tl.cut != 24 ||
-        P->npoints >= 2L * tl.n)
-        return P->tcur;
-    for (size_t i = 0; i < P->tlists.size(); ++i)
-        if (P->tlists[i].shape[0] == 8 && P->tlists[i].cut == 16) return (int)i;
-    return P->tcur;
+    if (P->ndim == 2)
+    {
+        const double n = P->npoints, t = tl.n;
+        const double line = t * std::sqrt(t) / (mode == IBAMR_SPREAD_OVERWRITE ? 1024 : 1536);
+        return P->tsparse.n > 0 && n < line ? P->tsparse : tl;
+    }
+    if (P->kernel == K_IB4 && P->precision == IBAMR_FP64 && mode == IBAMR_SPREAD_OVERWRITE && tl.cut == 24 &&
+        P->npoints < 2L * tl.n)
+        for (const TileList& t : P->tlists)
+            if (t.shape[0] == 8 && t.cut == 16) return t;
+    return tl;
 }
 
 int find_shape(const ibamr_plan* P, const int* shape)
@@ -383,8 +403,13 @@ int build_tile_lists(ibamr_plan* P)
     {
         if (!shape_admissible(P, sh)) continue;
         P->tlists.emplace_back();
-        const int rc = build_tiles(P, sh, P->tlists.back());
+        const int rc = build_tiles(P, sh, P->ndim == 3 ? spread_cut(P, sh) : S2_TILE, P->tlists.back());
         if (rc != IBAMR_OK) return rc;
+        if (P->ndim == 2 && P->tlists.back().n >= S2_MANY_TILES)
+        {
+            const int rc2 = build_tiles(P, sh, 2 * S2_TILE, P->tsparse);
+            if (rc2 != IBAMR_OK) return rc2;
+        }
     }
     if (P->tlists.empty()) return fail(IBAMR_ERR_INVALID, "drift_cells too large for the tile size");
     P->tcur = 0;
@@ -416,7 +441,7 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
         constexpr int KER = decltype(ker)::value;
         SpreadArgs<T> a{};
         fill_spread_args<T>(P, slot, F, X, mode, a);
-        const TileList& tl = P->tlists[spread_list(P, mode)];
+        const TileList& tl = spread_list(P, mode);
         a.tiles = tl.d;
         if (P->npoints > 0)
         {
@@ -509,7 +534,10 @@ int ibamr_plan_spread_ds(ibamr_plan* P, int slot, const void* F, const double* X
             return fail(IBAMR_ERR_INVALID, "internal: tile shape without a kernel");
         }
         else
-            hipLaunchKernelGGL((k_spread2<KER, T>), dim3(tl.n), dim3(64), 0, s, a);
+        {
+            const auto kernel = tl.cut == S2_TILE ? k_spread2<KER, T, 1> : k_spread2<KER, T, 2>;
+            hipLaunchKernelGGL(kernel, dim3(tl.n), dim3(64), 0, s, a);
+        }
         HIP_OK(hipGetLastError());
         if (t_end) HIP_OK(hipEventRecord(t_end, s));
         return IBAMR_OK;

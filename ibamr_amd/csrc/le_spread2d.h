@@ -1,26 +1,30 @@
 // le_spread2d.h -- 2-D spread kernel for gfx950 (included by le_spread.hip after
 // le_spread3d.h, whose SpreadArgs, static_for and uniform_double it uses).
 //
-// One wavefront owns an 8 x 8 tile of one array, one grid value per lane, summed in
-// FP64 in a register.  As in k_spread3b the points pass through three steps: 64
-// candidates of the reachable bins at a time are filtered by cell and position into
-// a ring in LDS; up to 64 ring entries are staged, one per lane (weights, F); the
+// One wavefront owns an 8 x 8 tile of one array (NV = 1), one grid value per lane, or
+// 16 x 16 (NV = 2, for few points on large levels), four values per lane 8 apart of
+// which a stencil covers at most one, summed in FP64 in registers.  As in k_spread3b the
+// points pass through three steps: 64 candidates of the reachable bins at a time are
+// filtered by cell and position into a ring in LDS; up to 64 ring entries are staged, one per lane (weights, F); the
 // staged points are then applied one after another, four at a time so that their
 // LDS reads overlap: per lane two weights, two products and one addition.  Points
 // come in the bins' order (bin y, image y, bin x, image x; rank), so every value's
 // order of summation is fixed whatever the tile.
-// Bound by the serial chain of a tile's points (latency; 2-D grids have few tiles).
+// Bound by the serial chain of a tile's points (latency; 2-D grids have few tiles), with
+// few points on a large level by the number of workgroups.
 #pragma once
 
 namespace
 {
 constexpr int S2_TILE = 8;
 
-template <int KER, typename T>
+template <int KER, typename T, int NV>
 __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
 {
     using KT = KernelTraits<KER>;
     constexpr int W = KT::W;
+    constexpr int TILE = S2_TILE * NV;
+    static_assert(W <= 8 && NV <= 2, "a stencil covers at most one of a lane's values along an axis");
     constexpr bool FP64 = sizeof(T) == 8;
     constexpr int NREC = 2 * W + 1;                  // x and y weights and F of a hit
     constexpr int ROW = NREC % 2 ? NREC : NREC + 1;  // odd: rows written by 64 lanes without bank conflicts
@@ -48,8 +52,8 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
         alo[d] = P.ilo[d] - a.gcw[d];
         ahi[d] = P.ihi[d] + a.gcw[d] + (d == axis ? 1 : 0);
         an[d] = ahi[d] - alo[d] + 1;
-        flo[d] = alo[d] + td.t[d] * S2_TILE;
-        fhi[d] = min(flo[d] + S2_TILE - 1, ahi[d]);
+        flo[d] = alo[d] + td.t[d] * TILE;
+        fhi[d] = min(flo[d] + TILE - 1, ahi[d]);
         if (a.mode == IBAMR_SPREAD_ACCUMULATE_INTERIOR)
         {
             flo[d] = max(flo[d], P.ilo[d]);
@@ -59,10 +63,12 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
     }
     if (flo[0] > fhi[0] || flo[1] > fhi[1]) return;  // tile wholly in the ghost region
     const int gx = flo[0] + x, gy = flo[1] + y;
-    const bool in = gx <= fhi[0] && gy <= fhi[1];
+    auto in = [&](int k) { return gx + 8 * (k % NV) <= fhi[0] && gy + 8 * (k / NV) <= fhi[1]; };  // value k of the lane
     T* __restrict__ arr = a.arrays[td.patch * a.narr + (a.side ? td.comp : 0)];
     if (!a.side) arr += (size_t)td.comp * an[0] * an[1];
-    T* const at = arr + (size_t)(gx - alo[0]) + (size_t)an[0] * (size_t)(gy - alo[1]);
+    auto at = [&](int k) {
+        return arr + (size_t)(gx + 8 * (k % NV) - alo[0]) + (size_t)an[0] * (size_t)(gy + 8 * (k / NV) - alo[1]);
+    };
     const int fcomp = td.comp;
 
     // cells whose points can reach the tile, inside the patch's Lagrangian ghost box
@@ -136,7 +142,9 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
     // (f.m4:1463); LDataManager::spread (interior mode) spreads into zeroed data and
     // adds the old values afterwards (LDataManager.cpp:594, 661-663)
     const bool from_old = a.mode == IBAMR_SPREAD_ACCUMULATE;
-    double acc = from_old && in ? (double)*at : 0.0;
+    double acc[NV * NV];
+#pragma unroll
+    for (int k = 0; k < NV * NV; ++k) acc[k] = from_old && in(k) ? (double)*at(k) : 0.0;
 
     const unsigned long long lt = (1ull << lane) - 1ull;
     const double vol = a.vol, rvol = a.rvol;
@@ -269,7 +277,7 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
             }
             if (!FP64) Fv = Fv * T(rvol);
             r[2 * W] = Fv;
-            if (b[0] > -W && b[0] < S2_TILE && b[1] > -W && b[1] < S2_TILE)
+            if (b[0] > -W && b[0] < TILE && b[1] > -W && b[1] < TILE)
                 place = (b[0] + 8) | (b[1] + 8) << 8 | (safe ? 0 : 1 << 16);
         }
         __syncthreads();
@@ -279,13 +287,17 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
         {
             double c[4];
             bool under[4];
+            int which[4];  // of the lane's values the one that the stencil covers
             bool slow = false;
 #pragma unroll
             for (int m = 0; m < 4; ++m)
             {
                 const int jm = j + m;  // < 64
                 const int pl = __builtin_amdgcn_readlane(place, jm);
-                const unsigned ix = (unsigned)(x + 8 - (pl & 0xff)), iy = (unsigned)(y + 8 - ((pl >> 8) & 0xff));
+                const int dx = x + 8 - (pl & 0xff), dy = y + 8 - ((pl >> 8) & 0xff);
+                const int kx = NV == 2 && dx < 0 ? 1 : 0, ky = NV == 2 && dy < 0 ? 1 : 0;
+                const unsigned ix = (unsigned)(dx + 8 * kx), iy = (unsigned)(dy + 8 * ky);
+                which[m] = kx + NV * ky;
                 under[m] = max(ix, iy) < (unsigned)W;
                 slow = slow || (pl >> 16);
                 const T* r = s_row + jm * ROW;
@@ -311,12 +323,16 @@ __global__ __launch_bounds__(64) void k_spread2(SpreadArgs<T> a)
                 }
             }
 #pragma unroll
-            for (int m = 0; m < 4; ++m) acc = under[m] ? acc + c[m] : acc;
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int k = 0; k < NV * NV; ++k) acc[k] = under[m] && which[m] == k ? acc[k] + c[m] : acc[k];
         }
         __syncthreads();
         qh = (qh + n) & (QCAP - 1);
         qn -= n;
     }
-    if (in) *at = (overwrite || from_old) ? (T)acc : (T)((double)*at + acc);
+#pragma unroll
+    for (int k = 0; k < NV * NV; ++k)
+        if (in(k)) *at(k) = (overwrite || from_old) ? (T)acc[k] : (T)((double)*at(k) + acc[k]);
 }
 } // namespace

@@ -481,7 +481,7 @@ int ibamr_plan_info(const ibamr_plan* plan, int* ntiles, int* tile, int* nbins);
  * selects another list (a HIP graph captured earlier keeps launching the shape
  * it captured, which stays valid).  Shapes (x, y, z extents; the first is the
  * default):
- *   2-D: 16 x 16, in pieces of 8 x 8.
+ *   2-D: 16 x 16, in pieces of 8 x 8, on large levels with few points whole.
  *   3-D FP64: 8 x 8 grid lines times 32 or 16 z values, or 16 x 4 grid lines
  *     times 32.  The z values are held in registers, in pieces: 16 each, but 8
  *     x 8 x 32 in pieces of 8 on levels of few tiles and of 24 on levels of very
