@@ -180,6 +180,7 @@ int ibamr_plan_destroy(ibamr_plan* P)
     dfree(P->patches_d);
     for (TileList& t : P->tlists)
         if (t.same < 0) dfree(t.d);
+    dfree(P->tfine.d);
     dfree(P->tsparse.d);
     dfree(P->wt_d);
     dfree(P->sb_owner_d);

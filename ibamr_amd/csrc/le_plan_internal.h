@@ -164,6 +164,8 @@ struct ibamr_plan
     PatchDev* patches_d = nullptr;
     std::vector<TileList> tlists;      // spread work lists, one per admissible tile shape (first: default)
     int tcur = 0;                      // the shape in use
+    TileList tfine;                    // FP64 3-D: the default shape in pieces of 8 (autotune builds it)
+    bool fine = false;                 // spreads with the default shape take tfine
     TileList tsparse;                  // 2-D levels of many tiles: whole 16 x 16 tiles (spread_list); n = 0: none
     // FP32C 3-D: the stencils of the bin-ordered positions, set up once per
     // spread (k_point_weights): for axis d and variant v (v = 1: x_lower - dx/2,

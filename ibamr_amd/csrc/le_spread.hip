@@ -356,7 +356,8 @@ int build_tiles(ibamr_plan* P, const Shape& sh, int cut, TileList& out)
     return IBAMR_OK;
 }
 
-// The work list a spread takes: the one chosen, but for few points per tile
+// The work list a spread takes: the one chosen, or its pieces of 8 where the autotuner
+// found them faster; but for few points per tile
 //   IB_4 3-D, fewer than two per tile of 24 values, overwriting: the list of 16 values:
 //     most tiles then write zeros, and those of IB_4 run four to a SIMD, whose
 //     unfinished lines of 24 planes no longer fit the L2 (512^3, 20000 points: 1.33 ms,
@@ -380,6 +381,7 @@ const TileList& spread_list(const ibamr_plan* P, int mode)
         const double line = t * std::sqrt(t) / (mode == IBAMR_SPREAD_OVERWRITE ? 1024 : 1536);
         return P->tsparse.n > 0 && n < line ? P->tsparse : tl;
     }
+    if (P->fine && (P->tcur == 0 || tl.same == 0)) return P->tfine;
     if (P->kernel == K_IB4 && P->precision == IBAMR_FP64 && mode == IBAMR_SPREAD_OVERWRITE && tl.cut == 24 &&
         P->npoints < 2L * tl.n)
         for (const TileList& t : P->tlists)
@@ -593,6 +595,7 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
     const bool timing = P->timing;
     P->timing = false;  // the trials are not the caller's launches
     const int start = P->tcur;
+    const bool start_fine = P->fine;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int best = start;
     float best_ms = std::numeric_limits<float>::infinity();
@@ -604,32 +607,56 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
         HIP_OK(hipEventCreate(&e0));
         HIP_OK(hipEventCreate(&e1));
         const size_t ns = P->tlists.size();
-        for (size_t i = 0; i < ns; ++i)
+        // FP64 3-D: the default shape is also tried in pieces of 8 values, whose shorter
+        // chains pay on crowded surfaces (131^3, 2.1 M points on a shell: IB_6 8.0 against
+        // 10.6 ms in pieces of 16, IB_4 4.8 against 7.0; spread over the volume 10 to 24 %
+        // slower): two sets of points that no rule on sizes tells apart.
+        const bool fine = P->ndim == 3 && P->precision == IBAMR_FP64 && P->tlists[0].shape[0] == 8 && P->tlists[0].cut > 8;
+        if (fine && !P->tfine.d)
         {
-            for (int d = 0; d < 3; ++d) shapes[3 * i + d] = P->tlists[i].shape[d];
-            ms[i] = std::numeric_limits<float>::infinity();
-            if (P->tlists[i].same >= 0) continue;
-            P->tcur = (int)i;
-            const int r = ibamr_plan_spread(P, slot, F, X, IBAMR_SPREAD_OVERWRITE, stream);  // untimed
+            const int* sh = P->tlists[0].shape;
+            const int r = build_tiles(P, Shape{sh[0], sh[1], sh[2]}, 8, P->tfine);
+            if (r != IBAMR_OK) return r;
+        }
+        float fine_ms = std::numeric_limits<float>::infinity();
+        auto trial = [&](size_t i, int n) -> int {  // i = ns: the default shape in pieces of 8
+            P->fine = i == ns;
+            P->tcur = i == ns ? 0 : (int)i;
+            for (int k = 0; k < n; ++k)
+            {
+                const int r = ibamr_plan_spread(P, slot, F, X, IBAMR_SPREAD_OVERWRITE, stream);
+                if (r != IBAMR_OK) return r;
+            }
+            return IBAMR_OK;
+        };
+        auto skip = [&](size_t i) { return i == ns ? !fine : P->tlists[i].same >= 0; };
+        for (size_t i = 0; i <= ns; ++i)
+        {
+            if (i < ns)
+            {
+                for (int d = 0; d < 3; ++d) shapes[3 * i + d] = P->tlists[i].shape[d];
+                ms[i] = std::numeric_limits<float>::infinity();
+            }
+            if (skip(i)) continue;
+            const int r = trial(i, 1);  // untimed
             if (r != IBAMR_OK) return r;
         }
         for (int round = 0; round < ROUNDS; ++round)
-            for (size_t i = 0; i < ns; ++i)
+            for (size_t i = 0; i <= ns; ++i)
             {
-                if (P->tlists[i].same >= 0) continue;
-                P->tcur = (int)i;
+                if (skip(i)) continue;
                 HIP_OK(hipEventRecord(e0, s));
-                for (int k = 0; k < reps; ++k)
-                {
-                    const int r = ibamr_plan_spread(P, slot, F, X, IBAMR_SPREAD_OVERWRITE, stream);
-                    if (r != IBAMR_OK) return r;
-                }
+                const int r = trial(i, reps);
+                if (r != IBAMR_OK) return r;
                 HIP_OK(hipEventRecord(e1, s));
                 HIP_OK(hipEventSynchronize(e1));
                 float t = 0.0f;
                 HIP_OK(hipEventElapsedTime(&t, e0, e1));
-                ms[i] = std::min(ms[i], t / reps);
+                float& m = i == ns ? fine_ms : ms[i];
+                m = std::min(m, t / reps);
             }
+        P->fine = fine_ms < ms[0];
+        ms[0] = std::min(ms[0], fine_ms);
         for (size_t i = 0; i < ns; ++i)  // a shared list has its owner's time
             if (P->tlists[i].same >= 0) ms[i] = ms[P->tlists[i].same];
         for (size_t i = 0; i < ns; ++i)
@@ -647,6 +674,7 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
     if (rc != IBAMR_OK)
     {
         P->tcur = start;
+        P->fine = start_fine;
         return rc;
     }
     *ncand = (int)P->tlists.size();

@@ -506,7 +506,9 @@ int ibamr_plan_info(const ibamr_plan* plan, int* ntiles, int* tile, int* nbins);
  *     untimed spread of F at X into the arrays
  *     bound to `slot` (IBAMR_SPREAD_OVERWRITE: their values are replaced), then
  *     3 rounds over all shapes of `reps` timed spreads each, and keeps the
- *     shape with the fastest round.  shapes[3*i .. 3*i+2] and ms[i] (capacity
+ *     shape with the fastest round.  FP64 3-D: the default shape is timed in
+ *     pieces of 8 values as well, its time is the smaller one, and spreads with
+ *     it take the faster pieces until the next autotune.  shapes[3*i .. 3*i+2] and ms[i] (capacity
  *     IBAMR_MAX_TILE_SHAPES) receive each candidate and its best round's mean
  *     time per spread call, *ncand their number; synchronises the stream.
  *     Points must be binned. */

@@ -63,3 +63,35 @@ def test_shapes_with_the_same_pieces(orc, n, shared):
         for a, b in zip(dev, want):
             assert np.array_equal(a.cpu().numpy(), b), sh
     plan.close()
+
+
+@pytest.mark.parametrize("kernel", ["IB_4", "IB_6", "BSPLINE_3"])
+def test_tuned_pieces(orc, kernel):
+    """Points crowded on a sphere, where pieces of 8 values are the faster ones: the same
+    bits after the autotuner's choice, in every mode, with every shape, and again after
+    tuning for few points."""
+    n, m = 104, 150000
+    rng = np.random.default_rng(m)
+    D = rng.standard_normal((m, 3))
+    X = 0.5 + 0.2 * D / np.linalg.norm(D, axis=1, keepdims=True)
+    F = rng.standard_normal(X.shape)
+    level = ia.Level.uniform_periodic(n, 3)
+    plan = ia.LevelPlan(level, kernel, ia.SIDE, ia.FP64, max_points=m)
+    f = [np.zeros(ia.array_shape(level, 0, plan.data_gcw, ia.SIDE, axis=a)) for a in range(3)]
+    for k in (m, 100):
+        want = _oracle_spread(orc, level, plan, f, X[:k], F[:k], kernel)
+        Xd, Fd = _dev(np.ascontiguousarray(X[:k])), _dev(np.ascontiguousarray(F[:k]))
+        dev = [_dev(a) for a in f]
+        plan.bind(0, dev)
+        plan.bin(Xd)
+        t = plan.autotune(0, Fd, Xd, reps=2)
+        assert t[(8, 8, 16)] == t[(8, 8, 32)] and plan.tile_shape == min(t, key=t.get)
+        for sh in t:
+            plan.tile_shape = sh
+            for mode in (ia.OVERWRITE, ia.ACCUMULATE):
+                for a in dev:
+                    a.fill_(0.0 if mode == ia.ACCUMULATE else 3.0)
+                plan.spread(0, Fd, Xd, mode=mode)
+                for a, b in zip(dev, want):
+                    assert np.array_equal(a.cpu().numpy(), b), (k, sh, mode)
+    plan.close()
