@@ -3,8 +3,9 @@
 //
 // Interpolation (k_interp3): one IBAMR_I3_THREADS-thread (512) workgroup per
 // superbin (2x2x2 bins = 16^3 cells) or half of one (interp3_cut).  For each array it
-// finds the exact stencil extent of its points, stages that block of the ghosted array into LDS with coalesced
-// loads, then each thread sums the W^3 stencil of its points from LDS.
+// finds the exact stencil extent of its points, stages that block of the ghosted array
+// into LDS with coalesced loads, then each thread sums the W^3 stencil of its points
+// from LDS.
 #pragma once
 
 namespace
@@ -33,10 +34,12 @@ constexpr int interp3_edge()
 //     the most it loses is a shell on 160^3, 420 / 392).  Not BSPLINE_6, whose weights
 //     take the time (200^3, 2 M uniform: 923 / 729);
 //   few superbins hold points, so that whole ones leave CUs idle or one of them is the
-//     last to end: up to 128 (256 CUs), or up to 768 of 1280 points and more on average
-//     (IB_4 40^3, 3000 points 17 / 21; 10^6 points on a shell 160^3 184 / 269, 256^3 140 /
-//     149; 512 k points in a ball 160^3 80 / 137), but for BSPLINE_6 between 128 and 256
-//     (one whole block a CU; 10^6 points on a shell 160^3 609 / 542).
+//     last to end: up to 256 (as many as CUs), or up to 768 of 1280 points and more on
+//     average (IB_4 40^3, 3000 points 17 / 21; 10^5 on a shell 160^3 34 / 45, 10^6 184 /
+//     269, 256^3 140 / 149; 92^3, 0.1 a cell uniform 21 / 23; 512 k points in a ball 160^3
+//     80 / 137).  BSPLINE_6 (one whole block a CU): up to 96 on larger levels, up to 128
+//     where the level has no more, and not between (128^3, 2000 points on a shell 59 / 35;
+//     10^6 on a shell 160^3 609 / 542).
 // Elsewhere whole superbins: IB_4, 0.03 points a cell uniform 128^3 37 / 25, 512^3 2258 /
 // 1457; 0.25 a cell 128^3 64 / 52, 200^3 254 / 210.  FP32C (three or four blocks fit as
 // they are) IB_6 512^3 1832 / 1394, IB_4 and BSPLINE_3 of a 384^3 level 231 / 217 and
@@ -49,7 +52,7 @@ constexpr int interp3_edge()
 template <int KER>
 __device__ __forceinline__ bool interp3_halves(int nactive, int npoints)
 {
-    return nactive <= 128 || (nactive > (KER == K_BS6 ? 256 : 128) && nactive <= 768 && npoints >= 1280 * nactive);
+    return nactive <= (KER == K_BS6 ? 96 : 256) || (nactive > 256 && nactive <= 768 && npoints >= 1280 * nactive);
 }
 
 // A cut superbin's block has 8 cells less along z.

@@ -95,7 +95,7 @@ enum InterpCut : int
 inline int interp3_cut(int kernel, int precision, int nsb)
 {
     if (precision != IBAMR_FP64 || kernel == K_PWL) return I3_WHOLE;
-    if (kernel == K_IB6 || nsb <= 128) return I3_HALVES;
+    if (kernel == K_IB6 || nsb <= (kernel == K_BS6 ? 128 : 256)) return I3_HALVES;
     return nsb <= 4096 ? I3_BY_POINTS : I3_WHOLE;
 }
 

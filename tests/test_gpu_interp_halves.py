@@ -1,6 +1,7 @@
 """FP64 interpolation from whole and from halved superbins on both sides of the
-rules that choose (125 superbins: halves; 216: by the points, which fill more than
-128 superbins, or a part of the level only; 4913: whole ones), bit for bit against
+rules that choose (125 superbins: halves; 216: halves, BSPLINE_6 by the points; 343:
+by the points, which fill more than 256 superbins, or a part of the level only; 4913:
+whole ones), bit for bit against
 the oracle: points on superbin and half-superbin faces, crowded cells, a level of
 one patch and one whose superbins several patches share."""
 import numpy as np
@@ -22,7 +23,7 @@ def _points(rng, n, part=1.0):
     return np.ascontiguousarray(np.clip(np.concatenate([X, D, E]), 0.0, np.nextafter(1.0, 0.0)))
 
 
-@pytest.mark.parametrize("n,part", [(80, 1.0), (88, 1.0), (88, 0.4)])
+@pytest.mark.parametrize("n,part", [(80, 1.0), (88, 1.0), (88, 0.4), (104, 1.0), (104, 0.4)])
 @pytest.mark.parametrize("kernel", ["IB_4", "IB_6", "BSPLINE_3", "BSPLINE_5", "BSPLINE_6", "PIECEWISE_LINEAR"])
 def test_one_patch(orc, n, part, kernel):
     print("interp halves", n, part, kernel, flush=True)
@@ -46,7 +47,7 @@ def test_more_superbins(orc):
 def test_binned_again(orc):
     """One plan, points that fill the level, then a part of it, in turn: each
     binning counts anew."""
-    n, kernel = 88, "BSPLINE_3"
+    n, kernel = 104, "BSPLINE_3"
     rng = np.random.default_rng(7)
     level = ia.Level.uniform_periodic(n, 3)
     plan = ia.LevelPlan(level, kernel, ia.SIDE, ia.FP64, max_points=4000)
@@ -61,7 +62,7 @@ def test_binned_again(orc):
     plan.close()
 
 
-@pytest.mark.parametrize("n", [80, 88])
+@pytest.mark.parametrize("n", [80, 88, 104])
 @pytest.mark.parametrize("kernel", ["IB_4", "BSPLINE_3"])
 def test_shared_superbins(orc, n, kernel):
     """Patches cut inside superbins: every point from the patch that owns its cell."""
