@@ -476,7 +476,7 @@ template <typename T>
 __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* flo, const int* fhi, int adjoint, long t)
 {
     const int nd = P.ndim;
-    int b[3] = {0, 0, 0}, s[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, n[3] = {1, 1, 1}, in[3] = {1, 1, 1};
+    int b[3] = {0, 0, 0}, s[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, n[3] = {1, 1, 1};
     for (int d = 0; d < nd; ++d)
     {
         const int up = (loc >> d) & 1;
@@ -484,9 +484,9 @@ __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* f
         s[d] = up ? 1 : -1;
         lo[d] = flo[d];
         n[d] = fhi[d] - flo[d] + 1;
-        in[d] = bd_inward(up, b[d], flo[d], fhi[d]);
     }
-    const int cube = in[0] * in[1] * in[2];
+    auto in = [&](int d) { return bd_inward(s[d] > 0, b[d], flo[d], fhi[d]); };
+    const int cube = in(0) * in(1) * (nd == 3 ? in(2) : 1);
     auto source = [&](int q, int* x, int* m) {
         x[0] = lo[0] + q % n[0], x[1] = lo[1] + (q / n[0]) % n[1], x[2] = lo[2] + q / (n[0] * n[1]);
         m[2] = 0;
@@ -518,8 +518,8 @@ __device__ void bd_cc_corner(const BPatch<T>& P, int comp, int loc, const int* f
         int r = (int)t;
         for (int d = 0; d < nd; ++d)
         {
-            y[d] = b[d] - s[d] * (r % in[d]);
-            r /= in[d];
+            y[d] = b[d] - s[d] * (r % in(d));
+            r /= in(d);
         }
     }
     else
