@@ -48,7 +48,9 @@ constexpr int interp3_edge()
 // are binned): where it decides (I3_BY_POINTS) twice the workgroups are launched and
 // the second half ends at once if superbins are taken whole.  Up to 4096 superbins
 // (256^3) that costs 1 % at most, at 512^3 (20000 points on a shell) 33 of 123 us; there
-// superbins are whole (10^6 points 244 / 202).
+// superbins are whole (10^6 points 244 / 202).  BSPLINE_3 with less than two points per
+// superbin differs by their layout (512^3, 32768 points uniform 800 / 975, on a shell
+// 138 / 121): whole.
 template <int KER>
 __device__ __forceinline__ bool interp3_halves(int nactive, int npoints)
 {
