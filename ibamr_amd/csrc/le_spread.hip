@@ -616,7 +616,12 @@ int ibamr_plan_autotune(ibamr_plan* P, int slot, const void* F, const double* X,
         {
             const int* sh = P->tlists[0].shape;
             const int r = build_tiles(P, Shape{sh[0], sh[1], sh[2]}, 8, P->tfine);
-            if (r != IBAMR_OK) return r;
+            if (r != IBAMR_OK)
+            {
+                if (P->tfine.d) (void)hipFree(P->tfine.d);  // not written: the next call builds it anew
+                P->tfine = TileList();
+                return r;
+            }
         }
         float fine_ms = std::numeric_limits<float>::infinity();
         auto trial = [&](size_t i, int n) -> int {  // i = ns: the default shape in pieces of 8
